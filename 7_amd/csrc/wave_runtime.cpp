@@ -20,6 +20,7 @@
 
 #include "attention.hpp"
 #include "gemm.hpp"
+#include "mxfp8_quant.hpp"
 
 namespace {
 
@@ -763,6 +764,25 @@ int wave_fa_fwd_mxfp8_launch(const void *Q, const void *Q_scale, const void *K,
   a.lse = lse;
   return hip_status(wave::attention::launch_fwd_fp8(a, static_cast<hipStream_t>(stream)),
                     "wave_fa_fwd_mxfp8_launch");
+}
+
+int wave_mxfp8_quantize_launch(const void *X, void *E, void *S, int64_t outer, int64_t n,
+                               int64_t inner, int x_dtype, void *stream) {
+  if (!X || !E || !S)
+    return fail(WAVE_ERR_INVALID, "mxfp8 quantize: null X, E or S");
+  if (outer <= 0 || n <= 0 || inner <= 0)
+    return fail(WAVE_ERR_INVALID, "mxfp8 quantize: outer=%lld n=%lld inner=%lld must be positive",
+                (long long)outer, (long long)n, (long long)inner);
+  if (!is_out_dtype(x_dtype))
+    return fail(WAVE_ERR_INVALID, "mxfp8 quantize: dtype %d is not f32/f16/bf16", x_dtype);
+  const int64_t lim = (int64_t)1 << 42;  // values; no device holds as many
+  if (outer > lim / n || outer * n > lim / inner)
+    return fail(WAVE_ERR_UNSUPPORTED, "mxfp8 quantize: problem too large");
+  if ((uintptr_t)X % (x_dtype == WAVE_F32 ? 4 : 2) != 0)
+    return fail(WAVE_ERR_INVALID, "mxfp8 quantize: X must be aligned to its elements");
+  return hip_status(wave::quant::launch_mxfp8(X, E, S, (size_t)outer, (size_t)n, (size_t)inner,
+                                              x_dtype, static_cast<hipStream_t>(stream)),
+                    "wave_mxfp8_quantize_launch");
 }
 
 int wave_fa_f32_launch(const void *Q, const void *K, const void *V, float *O,

@@ -9,6 +9,7 @@ failures raise runtime.WaveError.
 from __future__ import annotations
 
 import ctypes
+import math
 
 import torch
 
@@ -265,14 +266,47 @@ def _fa_shapes(q, k, v):
     return B, Hq, k.shape[1], S, D
 
 
+def _eager_device_tensor(x: torch.Tensor) -> bool:
+    """Whether x is a plain device tensor outside any tracing or transform, so
+    that its pointer is what the operation runs on."""
+    return (x.is_cuda and type(x) in (torch.Tensor, torch.nn.Parameter)
+            and not torch.compiler.is_compiling()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def _mxfp8_quantize_launch(x: torch.Tensor, dim: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """mxfp8_quantize through wave_mxfp8_quantize_launch: one pass over x."""
+    x = x.detach().contiguous()
+    shape = list(x.shape)
+    outer, n, inner = math.prod(shape[:dim]), shape[dim], math.prod(shape[dim + 1:])
+    elems = torch.empty(shape, dtype=torch.uint8, device=x.device)
+    shape[dim] = -(-n // 32)
+    scales = torch.empty(shape, dtype=torch.uint8, device=x.device)
+    with torch.cuda.device(x.device):
+        rt.check(rt.lib().wave_mxfp8_quantize_launch(
+            x.data_ptr(), elems.data_ptr(), scales.data_ptr(), outer, n, inner, _DT[x.dtype],
+            _stream(x)))
+    return elems, scales
+
+
 def mxfp8_quantize(x: torch.Tensor, dim: int = -1) -> tuple[torch.Tensor, torch.Tensor]:
     """OCP MX-FP8 encoding of x along `dim` (its size a multiple of 32, or
     padded with zeros to one): blocks of 32 elements share the e8m0 scale
     2^(floor(log2(amax)) - 8) (the OCP MX rule for e4m3, whose largest
     exponent is 8), and each element is x / scale rounded to e4m3, saturated at
-    +-448.  Returns (e4m3 bytes as uint8, x's shape; e8m0 bytes as uint8, x's
+    +-448.  Device f32 / f16 / bf16 tensors take one pass of a HIP kernel
+    (wave_mxfp8_quantize_launch); everything else, the same formula as tensor
+    operations, with the same bytes.  Returns (e4m3 bytes as uint8, x's shape; e8m0 bytes as uint8, x's
     shape with `dim` divided by 32, rounded up)."""
     dim = dim % x.dim()
+    if _eager_device_tensor(x) and x.dtype in _DT and x.numel() > 0:
+        return _mxfp8_quantize_launch(x, dim)
+    return _mxfp8_quantize_formula(x, dim)
+
+
+def _mxfp8_quantize_formula(x: torch.Tensor, dim: int) -> tuple[torch.Tensor, torch.Tensor]:
+    """mxfp8_quantize as tensor operations (any device, any dtype)."""
     xs = x.float().movedim(dim, -1)
     n = xs.shape[-1]
     nb = -(-n // 32)

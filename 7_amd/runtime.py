@@ -22,6 +22,7 @@ OK, ERR_INVALID, ERR_UNSUPPORTED, ERR_WORKSPACE = 0, -1, -2, -3
 _P = ctypes.c_void_p
 _I = ctypes.c_int
 _F = ctypes.c_float
+_L = ctypes.c_int64
 _SZ = ctypes.c_size_t
 
 _SIGNATURES = {
@@ -47,6 +48,7 @@ _SIGNATURES = {
     "wave_fa_fwd_lse_launch": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _F, _P]),
     "wave_fa_fwd_mxfp8_launch": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I,
                                       _I, _F, _P]),
+    "wave_mxfp8_quantize_launch": (_I, [_P, _P, _P, _L, _L, _L, _I, _P]),
     "wave_fa_bwd_launch": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
                                 _I, _I, _F, _P]),
     "wave_status_string": (ctypes.c_char_p, [_I]),

@@ -274,6 +274,18 @@ int wave_fa_fwd_mxfp8_launch(const void *Q, const void *Q_scale, const void *K,
                              int seq, int head_dim, int out_dtype, int causal, float scale,
                              void *stream);
 
+/* The encoding of those inputs: X [outer][n][inner] (contiguous, x_dtype f32,
+ * f16 or bf16) -> E, e4m3 bytes of the same layout, and S, e8m0 bytes
+ * [outer][ceil(n/32)][inner]: each block of 32 values along n shares the
+ * scale 2^(floor(log2(amax)) - 8) (the OCP MX rule for e4m3, whose largest
+ * exponent is 8) and each value is x / scale rounded to e4m3, saturated at
+ * +-448.  A block of zeros, or one with a NaN, has the scale 2^-127.  Any
+ * alignment; 16-byte aligned buffers run fastest.  Q, K of the forward:
+ * (batch * heads * seq, 128, 1); V: (batch * heads, seq, 128).  No
+ * counterpart in the reference. */
+int wave_mxfp8_quantize_launch(const void *X, void *E, void *S, int64_t outer, int64_t n,
+                               int64_t inner, int x_dtype, void *stream);
+
 /* ---- flash-attention backward --------------------------------------------
  * dQ, dK, dV of O = softmax(scale * Q K^T) V (causal and GQA as the forward;
  * dK, dV sum over the q heads of each KV head) from dO, O and the lse of

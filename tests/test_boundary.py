@@ -376,3 +376,17 @@ def test_kernel_abi_header_matches_code_objects(tmp_path):
             assert lds + 131072 > v["LDS_LIMIT"], name
         seen.add(prefix)
     assert seen == set(family), seen
+
+
+@pytest.mark.parametrize("kw,status", [
+    (dict(X=None), -1), (dict(S=None), -1), (dict(outer=0), -1), (dict(n=-1), -1),
+    (dict(inner=0), -1), (dict(dt=3), -1), (dict(X=17), -1), (dict(dt=0, X=18), -1),
+    (dict(outer=1 << 30, n=1 << 30), -2),
+])
+def test_mxfp8_quantize_rejects_bad_arguments(wave, kw, status):
+    L = wave.runtime.lib()
+    a = dict(X=16, E=32, S=64, outer=1, n=32, inner=1, dt=1)
+    a.update(kw)
+    st = L.wave_mxfp8_quantize_launch(a["X"], a["E"], a["S"], a["outer"], a["n"], a["inner"],
+                                      a["dt"], None)
+    assert st == status and L.wave_last_error()
