@@ -20,6 +20,7 @@ struct GemmArgs {
   void *counters = nullptr; // Stream-K per-tile arrival counters (zeroed)
   int workers = 0;          // > 0 selects the Stream-K kernel
   bool force_masked = false;
+  int cus = 256;            // compute units of the device, for the block choice
   // MXFP4 (in_dtype kMXFP4): A [M][K/2], B [N][K/2] packed fp4; e8m0 scales
   // group-major [K/32][M] and [K/32][N].
   const void *a_scale = nullptr;
@@ -40,28 +41,47 @@ int k_iterations(int K);
 hipError_t launch(const GemmArgs &args, hipStream_t stream);
 // MXFP4 scaled GEMM (gemm_mxfp4.hip): M, N % 256 == 0, K % 128 == 0.
 hipError_t launch_mxfp4(const GemmArgs &args, hipStream_t stream);
-// Short-M kernel (gemm_skinny.hip): M <= 128, K % 64 == 0, aligned.
-bool skinny_supported(const GemmArgs &args);
-hipError_t launch_skinny(const GemmArgs &args, hipStream_t stream);
-// Split-K short-M kernel (gemm_skinny.hip): `bn`-column CTAs over
-// `splits` K ranges, fp32 partials in `slots` (skinny_split_slot_bytes)
-// reduced in the launch by each column block's last arriver, through
-// `counters` (skinny_split_counter_count 64-bit words, 8-byte aligned, any
-// contents before the launch: a word counts only under the launch's
-// nonzero `epoch`; left zero).  skinny_split_plan: the plan for the shape
-// on `cus` CUs,
-// splits == 0 when the shape takes the unsplit kernel (pointers and C's
-// leading dimension are checked by skinny_supported).
+
+// The kernel `launch_auto` runs for a shape.  bm = 0: the 256x256 tiles
+// (Stream-K when workers > 0), else a bm x bn block over `splits` K ranges
+// (gemm_block.hpp).
+struct GemmPlan {
+  int bm = 0, bn = 0, splits = 1;
+  int workers = 0;
+};
+// Limits a caller's workspace puts on a split: fp32 partial slots and 64-bit
+// counter words (two a block).
+struct SplitLimits {
+  size_t slot_bytes = 0, counter_words = 0;
+};
+// vec4: K % 4 == 0 and A, B 8-byte aligned; workers: what Stream-K would run
+// with (0: not offered).
+GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, int workers,
+                   const SplitLimits &limits);
+bool rows_vec4(const GemmArgs &args);
+// A small-block launch: `slots` / `counters` for splits > 1 (any contents: a
+// counter word counts only under this launch's nonzero `epoch`; left zero),
+// and zero_words 64-bit words at `zero` left zero.
+struct BlockWorkspace {
+  float *slots = nullptr;
+  unsigned long long *counters = nullptr, *zero = nullptr;
+  size_t zero_words = 0;
+  uint32_t epoch = 0;
+};
+hipError_t launch_blocks(const GemmArgs &args, const GemmPlan &plan, const BlockWorkspace &ws,
+                         hipStream_t stream);
+
+// The workspace contract of the shape-driven entry point for M <= 128:
+// partial slots of `splits` x (128 x bn) fp32 per bn columns, then two 64-bit
+// words per bn columns, which every launch that is given them leaves zero.
+// splits == 0: no workspace.
 struct SplitPlan {
   int splits = 0;
   int bn = 128;
 };
-SplitPlan skinny_split_plan(int M, int N, int K, int cus);
-size_t skinny_split_slot_bytes(int N, const SplitPlan &plan);
-size_t skinny_split_counter_count(int N, const SplitPlan &plan);
-hipError_t launch_skinny_split(const GemmArgs &args, const SplitPlan &plan, float *slots,
-                               unsigned long long *counters, uint32_t epoch,
-                               hipStream_t stream);
+SplitPlan short_m_workspace(int M, int N, int K, int cus);
+size_t short_m_slot_bytes(int N, const SplitPlan &plan);
+size_t short_m_counter_count(int N, const SplitPlan &plan);
 
 } // namespace gemm
 } // namespace wave

@@ -1,11 +1,14 @@
 // gemm_dispatch.hip -- host-side selection of the GEMM kernel variant
 // (aligned DMA path vs masked path, dtype/layout, tiled vs Stream-K).
+#include "gemm_block.hpp"
 #include "gemm_kernels.hpp"
 
 #ifndef WAVE_GEMM_GROUP_M
 #define WAVE_GEMM_GROUP_M 4
 #endif
 
+#include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace wave {
@@ -25,6 +28,18 @@ namespace gemm {
   WAVE_GEMM_EXTERN(IN, kBF16, true)
 WAVE_GEMM_EXTERN_IN(kF16)
 WAVE_GEMM_EXTERN_IN(kBF16)
+
+namespace block {
+#define WAVE_BLOCK_EXTERN(IN, OUT)                                             \
+  extern template hipError_t launch_block<IN, OUT>(const BlockParams &, int,   \
+                                                   int, bool, bool, hipStream_t);
+WAVE_BLOCK_EXTERN(kF16, kF32)
+WAVE_BLOCK_EXTERN(kF16, kF16)
+WAVE_BLOCK_EXTERN(kF16, kBF16)
+WAVE_BLOCK_EXTERN(kBF16, kF32)
+WAVE_BLOCK_EXTERN(kBF16, kF16)
+WAVE_BLOCK_EXTERN(kBF16, kBF16)
+} // namespace block
 
 template <int IN, int OUT>
 static hipError_t launch_out(const Params &p, bool cm, bool sk, int mode,
@@ -86,9 +101,200 @@ hipError_t count_nonzero(const uint32_t *counters, size_t count, int *result,
 int tiles_for(int extent) { return (extent + kTile - 1) / kTile; }
 int k_iterations(int K) { return (K + kSKUnit - 1) / kSKUnit; }
 
+bool rows_vec4(const GemmArgs &g) {
+  return g.K % 4 == 0 && aligned_to(g.A, 8) && aligned_to(g.B, 8);
+}
+
+// ---- which kernel a shape takes --------------------------------------------
+// Each candidate's time is estimated (microseconds) and the least taken.  The
+// constants are a fit to measured launches: f16, one MI355X (256 CUs), three
+// operand sets in turn, 3400 random shapes (M, N 1 to 16384, K 32 to 16384,
+// half of them M <= 128) times every block size and 1 to 8 splits.  On those
+// shapes the choice is on average 2 % from the best candidate and never more
+// than 8 % slower than the 256x256 / 32-column kernels it chose between
+// before, 2.6 times as fast in the mean.
+//
+// A block's stage (64 of K) costs s0 on an idle chip and s1 with a CTA on
+// every CU (its DMA is bound by what a CU fetches, 80 to 110 GB/s); further
+// CTAs queue (s2 a stage, `round` a CTA).  A split's exchange costs e0 plus
+// what all partials cost to publish (e1 a MB) and the last arriver to read
+// (e2 a 16 KiB slot).  No candidate beats its operands' time from HBM (4.2
+// TB/s; 5.0 when CTAs work on different K ranges); the two limits meet
+// smoothly, so that of two HBM-bound candidates the one with the faster loop
+// wins.
+namespace {
+struct BlockCost {
+  int bm, bn;
+  float base, s0, s1, s2, round, e0, e1, e2;
+};
+constexpr BlockCost kBlocks[] = {
+    {128, 128, 4.10f, .328f, .514f, .531f, 4.46f, 2.08f, .152f, .362f},
+    {128, 64, 3.64f, .228f, .282f, .331f, 3.56f, 1.44f, .228f, .600f},
+    {64, 64, 3.18f, .151f, .184f, .185f, 1.40f, .843f, .273f, 1.02f},
+    {32, 64, 3.09f, .107f, .132f, .123f, 1.25f, .814f, .503f, 1.95f},
+    {32, 32, 3.13f, .0735f, .0789f, .0765f, 1.09f, .801f, .979f, 3.82f},
+};
+// Rows off 8 bytes (element-by-element loads through registers): a stage of
+// the 256x256 kernel, and of a 64x64 block alone on its CU or sharing it with
+// others (1000^2 x 1001 60.3 us in tiles, 15.8 in blocks; 2048^2 59.8 / 32.7;
+// 3000^2 62.8 / about 70).
+constexpr float kMaskedTile = 3.4f, kMaskedBlock = .8f, kMaskedShared = .46f;
+constexpr int kMaxSplits = 8;
+constexpr int kMinSplitStages = 4;  // stages a split keeps
+
+int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The cube of a block launch's estimate (the smooth maximum of its own time
+// and its operands' time from HBM, without the root).
+float block_cost3(const BlockCost &c, int64_t tiles, int64_t nk, int splits, int cus,
+                  float hbm_mb) {
+  const int64_t ctas = tiles * splits, stages = up(nk, splits), load = up(ctas, cus);
+  const float stage = ctas <= cus ? c.s0 + (c.s1 - c.s0) * (float)ctas / (float)cus
+                                  : c.s2 * (float)load;
+  float t = c.base + stage * (float)stages + (float)(load - 1) * c.round;
+  if (splits > 1)
+    t += c.e0 + c.e1 * (float)(ctas * (c.bm * c.bn)) * 4e-6f +
+         c.e2 * (float)((splits - 1) * (c.bm * c.bn / 4096.f));
+  const float hbm = c.base + hbm_mb / (splits > 1 ? 5.0f : 4.2f);
+  return t * t * t + hbm * hbm * hbm;
+}
+
+// 256x256 tiles: a stage costs 1.0 (up to a quarter of the chip busy) to 1.5
+// (all of it); ragged edges or a K remainder 3 more a launch.
+float tile_stage(float busy, bool vec4) {
+  return vec4 ? 1.0f + 0.5f * std::min(1.0f, std::max(0.0f, (busy - 0.25f) / 0.75f))
+              : kMaskedTile;
+}
+float cube(float t) { return t * t * t; }
+} // namespace
+
+GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, int workers,
+                   const SplitLimits &limits) {
+  GemmPlan plan;
+  // Block row and column numbers are ints with room for a block's edge; far
+  // smaller shapes fill the chip with 256x256 tiles.
+  if (M > (1 << 28) || N > (1 << 28))
+    return plan;
+  const int64_t nk = up(K, 64), big = up(M, 256) * up(N, 256), rounds = up(big, cus);
+  const bool ragged = M % 256 || N % 256 || K % 64;
+  float best = cube(7.f + (float)rounds * tile_stage((float)big / (float)(rounds * cus), vec4) *
+                              (float)nk + (float)(rounds - 1) * 4.f + (ragged ? 3.f : 0.f));
+  if (workers > 0) {
+    // Stream-K: a worker's share of the stages, and 32 for the counter fill,
+    // the publish and the reduction.
+    const float t = cube(32.f + (float)(big * nk) / (float)workers *
+                                    tile_stage((float)workers / (float)cus, vec4));
+    if (t < best) {
+      best = t;
+      plan.workers = workers;
+    }
+  }
+  const float hbm_mb = 2e-6f * (float)K * ((float)M + (float)N);
+  for (const BlockCost &c : kBlocks) {
+    const int64_t tiles = up(M, c.bm) * up(N, c.bn);
+    if (tiles > (1 << 24) || (!vec4 && (c.bm != 64 || c.bn != 64)))
+      continue;
+    for (int splits = 1; splits <= (vec4 ? kMaxSplits : 1); ++splits) {
+      if (splits > 1 &&
+          (K / 64 < splits * kMinSplitStages || tiles * splits > 2 * cus ||
+           (size_t)(tiles * splits * c.bm * c.bn) * sizeof(float) > limits.slot_bytes ||
+           (size_t)tiles * 2 > limits.counter_words))
+        break;
+      const float t =
+          vec4 ? block_cost3(c, tiles, nk, splits, cus, hbm_mb)
+               : cube(c.base + (float)nk * std::max(kMaskedBlock,
+                                                    kMaskedShared * (float)up(tiles, cus)));
+      if (t < best) {
+        best = t;
+        plan.bm = c.bm;
+        plan.bn = c.bn;
+        plan.splits = splits;
+        plan.workers = 0;
+      }
+    }
+  }
+  return plan;
+}
+
+SplitPlan short_m_workspace(int M, int N, int K, int cus) {
+  SplitPlan plan;
+  if (M > 128 || N < 1024 || K % 64 != 0 || (uint64_t)K * 2u * 128u >= (1ull << 32) ||
+      (uint64_t)N * K * 2u >= (1ull << 32))
+    return plan;
+  // Columns in blocks of 64 when they leave room for at least two splits on
+  // the device's CUs, else of 128; at most 4 splits (at least 2 when the
+  // columns fill the CUs 32 at a time), at least 8 stages of 64 a split;
+  // none when a split keeps less than 4096 of K (2048 where M > 96 and the
+  // columns fill the CUs 32 at a time).
+  const int nk = K / 64;
+  const int narrow = (N + 31) / 32;
+  for (int bn : {64, 128}) {
+    const int tiles = (N + bn - 1) / bn;
+    int s = std::min(cus / tiles, 4);
+    if (s < 2 && bn == 128 && narrow > cus)
+      s = 2;
+    while (s > 1 && nk < 8 * s)
+      --s;
+    if (s < 2)
+      continue;
+    const int ks = K / s;
+    if (ks < 2048 || (ks < 4096 && (M <= 96 || narrow < cus)))
+      return plan;
+    plan.splits = s;
+    plan.bn = bn;
+    return plan;
+  }
+  return plan;
+}
+
+size_t short_m_slot_bytes(int N, const SplitPlan &plan) {
+  return (size_t)((N + plan.bn - 1) / plan.bn) * plan.splits * 128 * plan.bn * sizeof(float);
+}
+
+size_t short_m_counter_count(int N, const SplitPlan &plan) {
+  return 2 * (size_t)((N + plan.bn - 1) / plan.bn);
+}
+
+hipError_t launch_blocks(const GemmArgs &g, const GemmPlan &plan, const BlockWorkspace &ws,
+                         hipStream_t stream) {
+  if (plan.bm == 0 || plan.splits < 1 ||
+      (plan.splits > 1 && (!ws.slots || !ws.counters || !ws.epoch || g.K / 64 < plan.splits)))
+    return hipErrorInvalidValue;
+  block::BlockParams p{};
+  p.A = static_cast<const uint16_t *>(g.A);
+  p.B = static_cast<const uint16_t *>(g.B);
+  p.C = g.C;
+  p.M = g.M;
+  p.N = g.N;
+  p.K = g.K;
+  p.ldc = g.col_major ? g.M : g.N;
+  p.c_vec_ok = aligned_to(g.C, 16) && (size_t)p.ldc * (g.out_dtype == kF32 ? 4 : 2) % 16 == 0;
+  p.splits = plan.splits;
+  p.slots = ws.slots;
+  p.counters = ws.counters;
+  p.epoch = ws.epoch;
+  p.zero = ws.zero;
+  p.zero_words = (uint32_t)ws.zero_words;
+  const bool vec4 = rows_vec4(g);
+  auto in = [&](auto tag) {
+    constexpr int IN = decltype(tag)::value;
+    if (g.out_dtype == kF32)
+      return block::launch_block<IN, kF32>(p, plan.bm, plan.bn, vec4, g.col_major, stream);
+    if (g.out_dtype == kF16)
+      return block::launch_block<IN, kF16>(p, plan.bm, plan.bn, vec4, g.col_major, stream);
+    return block::launch_block<IN, kBF16>(p, plan.bm, plan.bn, vec4, g.col_major, stream);
+  };
+  if (g.in_dtype == kF16)
+    return in(std::integral_constant<int, kF16>{});
+  return in(std::integral_constant<int, kBF16>{});
+}
+
 hipError_t launch(const GemmArgs &g, hipStream_t stream) {
-  if (g.workers == 0 && !g.force_masked && !g.packed && skinny_supported(g))
-    return launch_skinny(g, stream);
+  if (g.workers == 0 && !g.force_masked && !g.packed) {
+    const GemmPlan plan = gemm_plan(g.M, g.N, g.K, g.cus, rows_vec4(g), 0, SplitLimits{});
+    if (plan.bm)
+      return launch_blocks(g, plan, BlockWorkspace{}, stream);
+  }
   Params p{};
   p.A = static_cast<const uint16_t *>(g.A);
   p.B = static_cast<const uint16_t *>(g.B);

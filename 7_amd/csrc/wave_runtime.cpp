@@ -1,7 +1,7 @@
 // wave_runtime.cpp -- the C ABI of libwave_runtime.so (include/wave_runtime.h).
 //
 // Validates every request on the host before any HIP call, maps it onto the
-// kernels in gemm_kernels.hpp / attention_kernels.hpp / fa_small.hip, and
+// kernels in gemm_kernels.hpp / gemm_block.hpp / attention_kernels.hpp / fa_small.hip, and
 // reports failures as status codes plus a per-thread message.  Also carries
 // the reference's seven memref -> pointer shims (runtime/wave_runtime.cpp:
 // 27-74) unchanged in behaviour.
@@ -303,6 +303,9 @@ int wave_gemm_launch(const void *A, const void *B, void *C, int M, int N, int K,
   g.in_dtype = in_dtype;
   g.out_dtype = out_dtype;
   g.col_major = c_layout == WAVE_COL_MAJOR;
+  st = device_cus(&g.cus);
+  if (st != WAVE_OK)
+    return st;
   return hip_status(wave::gemm::launch(g, static_cast<hipStream_t>(stream)),
                     "wave_gemm_launch");
 }
@@ -446,11 +449,11 @@ int wave_gemm_auto_workspace_bytes(int M, int N, int K, size_t *bytes) {
   if (st != WAVE_OK)
     return st;
   const int workers = auto_workers(M, N, K, cus);
-  const wave::gemm::SplitPlan plan = wave::gemm::skinny_split_plan(M, N, K, cus);
+  const wave::gemm::SplitPlan plan = wave::gemm::short_m_workspace(M, N, K, cus);
   *bytes = 0;
   if (plan.splits > 0)
-    *bytes = wave::gemm::skinny_split_slot_bytes(N, plan) +
-             wave::gemm::skinny_split_counter_count(N, plan) * sizeof(uint64_t);
+    *bytes = wave::gemm::short_m_slot_bytes(N, plan) +
+             wave::gemm::short_m_counter_count(N, plan) * sizeof(uint64_t);
   if (workers > 0) {
     size_t scratch = 0, counters = 0;
     st = streamk_sizes(M, N, workers, &scratch, &counters);
@@ -475,42 +478,78 @@ int wave_gemm_auto_launch(const void *A, const void *B, void *C, int M, int N, i
     return st;
   if (workspace && (uintptr_t)workspace % 16 != 0)
     return fail(WAVE_ERR_INVALID, "gemm auto: workspace must be 16-byte aligned");
-  const wave::gemm::SplitPlan plan = wave::gemm::skinny_split_plan(M, N, K, cus);
-  if (plan.splits > 0) {
-    // Short M: the split-K short-M kernel when the workspace holds its
-    // partial slots and counters and the operands suit the short-M kernel;
-    // otherwise wave_gemm_launch (the unsplit short-M kernel or the tiled one).
-    const size_t slot_bytes = wave::gemm::skinny_split_slot_bytes(N, plan);
-    const size_t count = wave::gemm::skinny_split_counter_count(N, plan);
-    wave::gemm::GemmArgs g;
-    g.A = A;
-    g.B = B;
-    g.C = C;
-    g.M = M;
-    g.N = N;
-    g.K = K;
-    g.in_dtype = in_dtype;
-    g.out_dtype = out_dtype;
-    g.col_major = c_layout == WAVE_COL_MAJOR;
-    if (!workspace || workspace_bytes < slot_bytes + count * sizeof(uint64_t) ||
-        !wave::gemm::skinny_supported(g))
-      return wave_gemm_launch(A, B, C, M, N, K, in_dtype, out_dtype, c_layout, stream);
-    float *slots = static_cast<float *>(workspace);
-    auto *counters = reinterpret_cast<unsigned long long *>(static_cast<char *>(workspace) +
-                                                            slot_bytes);
-    // No counter fill: the kernel's counts carry this launch's epoch.
-    return hip_status(wave::gemm::launch_skinny_split(g, plan, slots, counters, next_epoch(),
-                                                      static_cast<hipStream_t>(stream)),
-                      "wave_gemm_auto_launch (split-K short-M)");
-  }
-  const int workers = auto_workers(M, N, K, cus);
+  // The workspace's layout is the entry point's contract: for M <= 128 the
+  // short-M slots and counter words, else Stream-K's slots and counters.  A
+  // split plan lives inside it; a smaller workspace leaves the unsplit plans.
+  const wave::gemm::SplitPlan short_m = wave::gemm::short_m_workspace(M, N, K, cus);
+  int workers = auto_workers(M, N, K, cus);
   size_t scratch = 0, counter_bytes = 0;
-  if (workers > 0) {
+  if (short_m.splits > 0) {
+    scratch = wave::gemm::short_m_slot_bytes(N, short_m);
+    counter_bytes = wave::gemm::short_m_counter_count(N, short_m) * sizeof(uint64_t);
+  } else if (workers > 0) {
     st = streamk_sizes(M, N, workers, &scratch, &counter_bytes);
     if (st != WAVE_OK)
       return st;
   }
-  if (workers == 0 || !workspace || workspace_bytes < scratch + counter_bytes)
+  const bool have = scratch > 0 && workspace && workspace_bytes >= scratch + counter_bytes;
+  if (!have)
+    workers = 0;
+  wave::gemm::GemmArgs g;
+  g.A = A;
+  g.B = B;
+  g.C = C;
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.in_dtype = in_dtype;
+  g.out_dtype = out_dtype;
+  g.col_major = c_layout == WAVE_COL_MAJOR;
+  g.cus = cus;
+  // Short M: counters where the contract puts them.  Stream-K's workspace:
+  // two words a block taken from the top of the slots.
+  wave::gemm::SplitLimits limits;
+  char *counter_base = static_cast<char *>(workspace) + scratch;
+  if (have && short_m.splits > 0) {
+    limits.slot_bytes = scratch;
+    limits.counter_words = counter_bytes / sizeof(uint64_t);
+  } else if (have) {
+    constexpr size_t kWords = 4096;
+    limits.slot_bytes = scratch - kWords * sizeof(uint64_t);
+    limits.counter_words = kWords;
+    counter_base -= kWords * sizeof(uint64_t);
+  }
+  const wave::gemm::GemmPlan plan =
+      wave::gemm::gemm_plan(M, N, K, cus, wave::gemm::rows_vec4(g), workers, limits);
+  if (plan.bm) {
+    wave::gemm::BlockWorkspace ws;
+    if (plan.splits > 1) {
+      ws.slots = static_cast<float *>(workspace);
+      ws.counters = reinterpret_cast<unsigned long long *>(counter_base);
+      ws.epoch = next_epoch();
+    }
+    if (have && short_m.splits > 0) {
+      // Words no block counts on: the kernel clears them.
+      const size_t used =
+          plan.splits > 1 ? 2 * ((size_t)((M - 1) / plan.bm + 1) * ((N - 1) / plan.bn + 1)) : 0;
+      ws.zero = reinterpret_cast<unsigned long long *>(counter_base) + used;
+      ws.zero_words = limits.counter_words - used;
+    }
+    return hip_status(
+        wave::gemm::launch_blocks(g, plan, ws, static_cast<hipStream_t>(stream)),
+        "wave_gemm_auto_launch (blocks)");
+  }
+  if (have && short_m.splits > 0) {
+    // 256x256 tiles: clear the contract's words with a fill kernel.
+    st = hip_status(wave::gemm::zero_counters(reinterpret_cast<uint32_t *>(counter_base),
+                                              counter_bytes / sizeof(uint32_t),
+                                              static_cast<hipStream_t>(stream)),
+                    "wave_gemm_auto_launch: counter reset");
+    if (st != WAVE_OK)
+      return st;
+  }
+  workers = plan.workers;
+  if (workers == 0)
     return wave_gemm_launch(A, B, C, M, N, K, in_dtype, out_dtype, c_layout, stream);
   float *slots = static_cast<float *>(workspace);
   uint32_t *counters = reinterpret_cast<uint32_t *>(static_cast<char *>(workspace) + scratch);

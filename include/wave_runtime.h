@@ -144,23 +144,23 @@ int wave_gemm_streamk_counters_check(const uint32_t *counters, int M, int N,
 /* ---- shape-driven GEMM dispatch ------------------------------------------
  * No kernel symbol of the reference: the reference's harness picks its
  * tiled or Stream-K kernel per run (tools/wave-matmul-calibrate/
- * wave-matmul-perf-sweep.py:151-326 kernel matrix).  This entry point picks
- * for the caller: the tiled kernel (or, for M <= 128, the short-M kernel,
- * split over K into 2 to 4 ranges of 128-column blocks when N / 128 leaves
- * CUs idle: fp32 partials reduced in the launch by each block's last
- * arriver), or Stream-K with 2 * tiles workers when the 256x256 output tiles would leave
- * at least half the CUs idle (tiles <= CUs / 2) and K >= 4096 (K >= 8192
- * at exactly CUs / 2 tiles); with at most CUs / 4 tiles,
- * max(2 * tiles, min(tiles * (K / 2048), CUs / 2)) workers.  Stream-K
- * and the split short-M kernel take their workspace from `workspace`
- * (caller-owned, 16-byte aligned device memory of
- * wave_gemm_auto_workspace_bytes(M, N, K) bytes, 0 when the shape takes an
- * unsplit path; no initialisation needed: a Stream-K launch zeroes the
- * counters it uses with a fill kernel, and the split short-M kernel's
- * counters carry a per-launch tag, so whatever they hold counts as zero,
- * and it leaves them zero); with a smaller workspace the unsplit kernel
- * runs.  One launch in flight per workspace.  Same C as wave_gemm_launch
- * (c_layout row- or column-major). */
+ * wave-matmul-perf-sweep.py:151-326 kernel matrix).  wave_gemm_launch picks
+ * between 256x256 tiles and smaller blocks (32x32 to 128x128) by the time it
+ * expects of each; this entry point adds the kernels that need a workspace:
+ * the blocks with K split over 2 to 8 CTAs (fp32 partials summed in split
+ * order by each block's last arriver) and Stream-K, offered with 2 * tiles
+ * workers when the 256x256 output tiles would leave at least half the CUs
+ * idle (tiles <= CUs / 2) and K >= 4096 (K >= 8192 at exactly CUs / 2 tiles;
+ * with at most CUs / 4 tiles, max(2 * tiles, min(tiles * (K / 2048),
+ * CUs / 2)) workers).  `workspace` is caller-owned, 16-byte aligned device
+ * memory of wave_gemm_auto_workspace_bytes(M, N, K) bytes (0 when the shape
+ * takes an unsplit path); it needs no initialisation: a Stream-K launch zeroes
+ * the counters it uses with a fill kernel, and a split block's counters carry
+ * a per-launch tag, so whatever they hold counts as zero.  For M <= 128 the
+ * workspace ends in two 64-bit words per column block, which every launch
+ * leaves zero.  With a smaller workspace an unsplit kernel runs.  One launch
+ * in flight per workspace.  Same C as wave_gemm_launch (c_layout row- or
+ * column-major). */
 int wave_gemm_auto_workspace_bytes(int M, int N, int K, size_t *bytes);
 int wave_gemm_auto_launch(const void *A, const void *B, void *C, int M, int N,
                           int K, int in_dtype, int out_dtype, int c_layout,
