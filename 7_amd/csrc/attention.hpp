@@ -28,6 +28,8 @@ hipError_t launch_fwd(const FwdArgs &args, hipStream_t stream);
 // Backward (attention_bwd.hip): dQ, dK, dV of O = softmax(scale Q K^T) V from
 // dO, O and the forward's lse.  Layouts as FwdArgs (seq_q = seq_k = seq);
 // delta: caller scratch [batch][q_heads][seq] floats.  seq % 64 == 0.
+// workspace: bwd_workspace_bytes() for the dK/dV work split (16-byte aligned,
+// any contents); without it every key block is one CTA's.
 struct BwdArgs {
   const void *Q = nullptr, *K = nullptr, *V = nullptr, *O = nullptr, *dO = nullptr;
   const float *lse = nullptr;  // [batch][q_heads][seq]: ln sum_k exp(scale q.k)
@@ -37,7 +39,11 @@ struct BwdArgs {
   int dtype = 1;
   int causal = 0;
   float scale = 0.f;           // 0 selects 1/sqrt(128)
+  void *workspace = nullptr;
+  size_t workspace_bytes = 0;
+  int cus = 256;               // compute units of the device
 };
+size_t bwd_workspace_bytes(int batch, int q_heads, int kv_heads, int seq, bool causal, int cus);
 hipError_t launch_bwd(const BwdArgs &args, hipStream_t stream);
 
 // Block-scaled FP8 forward (attention_fwd8.hip): Q, K, V e4m3 bytes in the

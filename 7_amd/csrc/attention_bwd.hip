@@ -13,16 +13,17 @@
 // formulas above (oracle.py fa_backward) that is itself checked against
 // torch autograd.
 //
-// Three kernels, deterministic (no atomics):
+// Three or four kernels, deterministic (no atomics):
 //  * bwd_delta_kernel: -delta[row] = -sum_d dO[row][d] * O[row][d] in fp32
 //    (into the caller's scratch).
-//  * bwd_kv_pp_kernel (seq a multiple of 128): one CTA (8 waves, two groups
-//    of 4 one segment apart) per 128-key block of one KV head; it loops over
-//    the query blocks of every q head of the group (causal: the blocks at or
-//    after the key block), with each block's Q, dO, lse and -delta arriving
-//    by LDS DMA, and accumulates dK, dV in registers.  bwd_kv_kernel (one
-//    CTA of 4 waves per 64-key block, Q and dO staged through registers)
-//    covers seq = 64 (mod 128).
+//  * bwd_kv_pp_kernel: one CTA (8 waves, two groups of 4 one segment apart)
+//    per 128-key block of one KV head (the last block's second half may lie
+//    past the sequence); it loops over the query blocks of every q head of the
+//    group (causal: the blocks at or after the key block), with each block's
+//    Q, dO, lse and -delta arriving by LDS DMA, and accumulates dK, dV in
+//    registers.  Where those blocks are fewer than the CUs, or causal ones of
+//    uneven length, a block's loop is cut into chunks for several CTAs, which
+//    leave fp32 partials that bwd_kv_sum_kernel adds in chunk order.
 //  * bwd_q_kernel: one CTA per 64-query block of one q head; it loops over
 //    the key blocks (causal: up to the diagonal) and accumulates dQ.
 // Every product is an "NT" product C[m][n] = sum_k A[m][k] B[n][k] of 32x32
@@ -35,8 +36,7 @@
 // between the score products and the gradient products.  LDS tiles are
 // unpadded with XOR-swizzled 16-byte chunks (swz below), conflict-free for
 // every read these kernels make: 130 KiB (bwd_kv_pp_kernel, one CTA per
-// CU), 48 KiB (bwd_kv_kernel) and 40 KiB (dQ) of LDS, two CTAs per CU
-// (register-bound).
+// CU) and 72 KiB (dQ) of LDS, two CTAs per CU.
 #include "attention.hpp"
 #include "wave_common.hpp"
 
@@ -76,6 +76,10 @@ struct BwdParams {
   float scale;        // softmax scale
   float scale_log2;   // scale * log2(e)
   float inv_scale;    // 1 / scale
+  // dK/dV work split: chunks of at most `chunk` items (0: one CTA a block),
+  // `per_head` CTAs a KV head, partials [CTA][16][512] f32x4.
+  int chunk, per_head;
+  f32x4 *part;
 };
 
 // Two NT products over K = 128 that share their A rows: c0 += A0 . b0^T and
@@ -213,38 +217,12 @@ __device__ __forceinline__ void load_frags(const uint16_t *row, u32x4 (&f)[8]) {
     f[kk] = *reinterpret_cast<const u32x4 *>(row + 16 * kk + 8 * (lane >> 5));
 }
 
-// A [64][128] block of rows (row stride 128 elements) in flight through
-// registers: fetch() issues the global loads, put() writes the rows to LDS
-// (wide tile R).
-// Thread t handles row pairs x 16-byte chunks: unit u = t + 256*i, row pair
-// u / 16, chunk u % 16.
-struct BlockRegs {
-  u32x4 a[2], b[2];
-  __device__ __forceinline__ void fetch(const uint16_t *src) {
-    const uint32_t t = threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const uint32_t u = t + 256u * i, rp = u >> 4, c = u & 15u;
-      a[i] = *reinterpret_cast<const u32x4 *>(src + (size_t)(2 * rp) * kBD + 8 * c);
-      b[i] = *reinterpret_cast<const u32x4 *>(src + (size_t)(2 * rp + 1) * kBD + 8 * c);
-    }
-  }
-  __device__ __forceinline__ void put(uint8_t *R) const {
-    const uint32_t t = threadIdx.x;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const uint32_t u = t + 256u * i, rp = u >> 4, c = u & 15u;
-      *reinterpret_cast<u32x4 *>(R + toff<256>(2 * rp, 16 * c)) = a[i];
-      *reinterpret_cast<u32x4 *>(R + toff<256>(2 * rp + 1, 16 * c)) = b[i];
-    }
-  }
-};
-
 // CTA id -> work index with the CTAs of one head on one XCD (the
 // dispatcher places workgroup i on XCD i % 8), so they share that head's
 // K/V or Q/dO rows in the XCD's L2.
 __device__ __forceinline__ int xcd_pid(int raw, int total) {
-  return (total & 7) == 0 ? (raw & 7) * (total >> 3) + (raw >> 3) : raw;
+  const int xcd = raw & 7;  // the first total % 8 XCDs hold one more
+  return xcd * (total >> 3) + min(xcd, total & 7) + (raw >> 3);
 }
 
 // Store a 32x32 fp32 accumulator tile (rows row0.., columns col0..) of a
@@ -286,122 +264,37 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(BwdParams p, int rows) {
     p.delta[row] = -s;
 }
 
-// dK, dV of one 64-key block of one KV head.
-template <int DT, bool CAUSAL>
-__global__ __launch_bounds__(256, 2) void bwd_kv_kernel(BwdParams p) {
-  __shared__ __attribute__((aligned(16))) uint8_t smem[2 * kWide + 2 * kNarrowS];
-  uint8_t *sQ = smem, *sdO = sQ + kWide, *sPt = sdO + kWide, *sdSt = sPt + kNarrowS;
-  const int nb = p.seq / kBlk;
-  const int pid = xcd_pid((int)blockIdx.x, (int)gridDim.x);
-  const int kb = pid % nb, bhk = pid / nb;
-  const int b = bhk / p.kv_heads, hkv = bhk - b * p.kv_heads;
-  const int group = p.q_heads / p.kv_heads;
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const size_t kv_off = ((size_t)bhk * p.seq + (size_t)kb * kBlk) * kBD;
+// Work items of 128-key block kb2 of a KV head: (q head of the group, 64-query
+// block); causal: the blocks at or after the key block.
+__host__ __device__ __forceinline__ int kv_items(int group, int nb, int kb2, bool causal) {
+  return group * (nb - (causal ? 2 * kb2 : 0));
+}
+__host__ __device__ __forceinline__ int kv_chunks(int items, int chunk) {
+  return chunk > 0 ? (items + chunk - 1) / chunk : 1;
+}
 
-  // Score tiles: wave w computes S[q][key] for q half w&1, key half w>>1;
-  // lane l holds key kh2*32 + l%32 and queries qh2*32 + 8g + 4(l/32) + e.
-  const int qh2 = wave & 1, kh2 = wave >> 1;
-  // Gradient tiles: key half w&1, d quarters 2(w>>1), 2(w>>1)+1.
-  const int kh = wave & 1, dq = wave >> 1;
-  // K and V rows of this wave's key half as B fragments, for the whole CTA.
-  u32x4 kf[8], vf[8];
-  load_frags(p.K + kv_off + (size_t)(kh2 * 32 + (lane & 31)) * kBD, kf);
-  load_frags(p.V + kv_off + (size_t)(kh2 * 32 + (lane & 31)) * kBD, vf);
-  // Gradient accumulators: dV columns (2 dq) * 32 and (2 dq + 1) * 32, then
-  // dK's.
-  f32x16 g[4] = {f32x16{}, f32x16{}, f32x16{}, f32x16{}};
-  const int key = kb * kBlk + kh2 * 32 + (int)(lane & 31);
-  // Work items: (q head h of the group, query block qb), h major (causal:
-  // the blocks at or after the key block); the next item's Q and dO rows
-  // and its lse / delta are fetched while this one's products run.
-  const int qb0 = CAUSAL ? kb : 0, items = group * (nb - qb0);
-  auto rows_of = [&](int h, int q) {  // first row of item (h, q) in [B*Hq*S]
-    return ((size_t)b * p.q_heads + (size_t)hkv * group + h) * p.seq + (size_t)q * kBlk;
-  };
-  // This wave's score rows of an item: lse and -delta of rows
-  // qh2*32 + 8 g + 4 (l / 32) + e as the accumulators' start values.
-  f32x16 s, dp;
-  auto load_stats = [&](size_t rb) {
-    const size_t r0 = rb + qh2 * 32 + 4 * (lane >> 5);
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      const f32x4 a = *reinterpret_cast<const f32x4 *>(p.lse + r0 + 8 * g4);
-      const f32x4 d = *reinterpret_cast<const f32x4 *>(p.delta + r0 + 8 * g4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        s[4 * g4 + e] = a[e];
-        dp[4 * g4 + e] = d[e];
-      }
-    }
-  };
-  int h = 0, qb = qb0;
-  BlockRegs rq, rdo;
-  rq.fetch(p.Q + rows_of(0, qb0) * kBD);
-  rdo.fetch(p.dO + rows_of(0, qb0) * kBD);
-  load_stats(rows_of(0, qb0));
-  for (int it = 0; it < items; ++it) {
-    int hn = h, qbn = qb + 1;
-    if (qbn == nb) {
-      qbn = qb0;
-      ++hn;
-    }
-    const bool more = it + 1 < items;
-    __syncthreads();  // the previous item's readers are done
-    rq.put(sQ);
-    rdo.put(sdO);
-    if (more) {
-      rq.fetch(p.Q + rows_of(hn, qbn) * kBD);
-      rdo.fetch(p.dO + rows_of(hn, qbn) * kBD);
-    }
-    // The score accumulator starts at -lse / scale and dP's at -delta, so
-    // exp2(c * s) = P and dp = dP - delta after the products.
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      s[r] *= -p.inv_scale;
-    __syncthreads();
-    mma2_nt_reg<DT>(s, sQ, kf, dp, sdO, vf, qh2 * 32);
-    // P and dS; P^T / dS^T rows = keys, 4 consecutive queries per store.
-#pragma unroll
-    for (int g4 = 0; g4 < 4; ++g4) {
-      float pv[4], dsv[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = 4 * g4 + e;
-        const int q = qb * kBlk + qh2 * 32 + 8 * g4 + 4 * (int)(lane >> 5) + e;
-        float pr = __builtin_amdgcn_exp2f(s[r] * p.scale_log2);
-        if (CAUSAL && key > q)
-          pr = 0.f;
-        pv[e] = pr;
-        dsv[e] = pr * dp[r];
-      }
-      const uint32_t off =
-          toff<128>(kh2 * 32 + (lane & 31), 2 * (qh2 * 32 + 8 * g4 + 4 * (lane >> 5)));
-      *reinterpret_cast<u32x2 *>(sPt + off) = u32x2{pack2<DT>(pv[0], pv[1]), pack2<DT>(pv[2], pv[3])};
-      *reinterpret_cast<u32x2 *>(sdSt + off) =
-          u32x2{pack2<DT>(dsv[0], dsv[1]), pack2<DT>(dsv[2], dsv[3])};
-    }
-    __syncthreads();
-    const uint8_t *const ga[2] = {sPt, sdSt};
-    const uint8_t *const gr[2] = {sdO, sQ};
-    mma_grad<DT, 2>(g, ga, kh * 32, gr, (2 * dq) * 32, (2 * dq + 1) * 32);
-    if (more)
-      load_stats(rows_of(hn, qbn));
-    h = hn;
-    qb = qbn;
+// CTA c (0 .. per_head-1) of a KV head -> its block, its chunk of the block's
+// items and how many the block has.
+struct KvChunk {
+  int kb2, index, count;
+};
+template <bool CAUSAL>
+__device__ __forceinline__ KvChunk kv_chunk(const BwdParams &p, int group, int nb, int c) {
+  if (!CAUSAL || p.chunk == 0) {
+    const int n = kv_chunks(group * nb, p.chunk);
+    return {c / n, c % n, n};
   }
-  uint16_t *dK = p.dK + kv_off, *dV = p.dV + kv_off;
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    store_tile32<DT>(dV, kh * 32, (2 * dq + t) * 32, g[t], 1.f);
-    store_tile32<DT>(dK, kh * 32, (2 * dq + t) * 32, g[2 + t], p.scale);
+  for (int kb2 = 0;; ++kb2) {
+    const int n = kv_chunks(kv_items(group, nb, kb2, true), p.chunk);
+    if (c < n)
+      return {kb2, c, n};
+    c -= n;
   }
 }
 
 // dK, dV of a 128-key block of one KV head as two groups of four waves:
-// group g (waves 4g .. 4g+3) owns keys 64 g .. 64 g + 63 of the block and
-// does for them what bwd_kv_kernel does for its 64 keys (same wave roles,
-// same products), on the same work items.  The groups share each item's Q
+// group g (waves 4g .. 4g+3) owns keys 64 g .. 64 g + 63 of the block, on
+// the same work items.  The groups share each item's Q
 // and dO rows and its rows' lse and -delta, which arrive by LDS DMA into a
 // 3-buffer ring (so no global load is waited for inside the loop), and run
 // one segment apart ("ping-pong"), so that on every SIMD one wave's MFMAs
@@ -435,19 +328,23 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
   // and -delta (256 B each).
   constexpr uint32_t kStats = 2 * kWide, kQD = kStats + 512;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[3 * kQD + 4 * kNarrowS];
-  const int nb = p.seq / kBlk, nkb = nb / 2;
+  const int nb = p.seq / kBlk;
   const int pid = xcd_pid((int)blockIdx.x, (int)gridDim.x);
-  const int kb2 = pid % nkb, bhk = pid / nkb;
+  const int bhk = pid / p.per_head;
   const int b = bhk / p.kv_heads, hkv = bhk - b * p.kv_heads;
   const int group = p.q_heads / p.kv_heads;
   const uint32_t wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const uint32_t grp = wave >> 2, wg = wave & 3;
-  const int kb = 2 * kb2 + (int)grp;  // this group's 64-key block
+  const KvChunk chunk = kv_chunk<CAUSAL>(p, group, nb, pid - bhk * p.per_head);
+  const int kb2 = chunk.kb2;
+  // This group's 64-key block; past the sequence (the last block's second half
+  // when nb is odd) it repeats the last one and stores nothing.
+  const bool keys_in = 2 * kb2 + (int)grp < nb;
+  const int kb = keys_in ? 2 * kb2 + (int)grp : nb - 1;
   const size_t kv_off = ((size_t)bhk * p.seq + (size_t)kb * kBlk) * kBD;
   uint8_t *sPt = smem + 3 * kQD + grp * 2 * kNarrowS, *sdSt = sPt + kNarrowS;
   const uint32_t lds0 = lds_addr(smem);
-  // Wave roles within the group, as in bwd_kv_kernel.
-  // Score products: query half qh2, key half kh2.  Gradient products: wave
+  // Wave roles within the group.  Score products: query half qh2, key half kh2.  Gradient products: wave
   // role 0 accumulates dV, role 1 dK, each for all 64 keys of the group and
   // d columns 64 dq .. 64 dq + 63.
   const int qh2 = wg & 1, kh2 = wg >> 1, role = wg & 1, dq = wg >> 1;
@@ -458,7 +355,9 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
   const int key = kb * kBlk + kh2 * 32 + (int)(lane & 31);
   // Work items (q head h, query block qb), h major; causal: the blocks at
   // or after group 0's key block (group 1's first one is wholly masked).
-  const int qb0 = CAUSAL ? 2 * kb2 : 0, items = group * (nb - qb0);
+  const int qb0 = CAUSAL ? 2 * kb2 : 0, block_items = group * (nb - qb0);
+  const int first = block_items * chunk.index / chunk.count;
+  const int items = block_items * (chunk.index + 1) / chunk.count - first;
   struct Cursor {
     int h, qb;
   };
@@ -506,7 +405,7 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
       }
     }
   };
-  Cursor dmac{0, qb0}, cur{0, qb0};
+  Cursor dmac{first / (nb - qb0), qb0 + first % (nb - qb0)}, cur = dmac;
   if (grp == 1)
     dma_item(dmac, 0);
   advance(dmac);
@@ -565,6 +464,18 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
     else
       lds_barrier();
   }
+  if (chunk.count > 1) {
+    f32x4 *part = p.part + (size_t)pid * (16 * 512) + threadIdx.x;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        part[(4 * t + r) * 512] =
+            f32x4{g[t][4 * r], g[t][4 * r + 1], g[t][4 * r + 2], g[t][4 * r + 3]};
+    return;
+  }
+  if (!keys_in)
+    return;
   uint16_t *dst = (role ? p.dK : p.dV) + kv_off;
   const float sc = role ? p.scale : 1.f;
 #pragma unroll
@@ -572,6 +483,42 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
 #pragma unroll
     for (int t = 0; t < 2; ++t)
       store_tile32<DT>(dst, a * 32, (2 * dq + t) * 32, g[2 * a + t], sc);
+}
+
+// dK, dV of the blocks that bwd_kv_pp_kernel cut into chunks: the partials'
+// sum in chunk order, rounded once.  One CTA a 32x32 tile set t (0 .. 3) of a
+// block, its threads standing for that kernel's.
+template <int DT, bool CAUSAL>
+__global__ __launch_bounds__(512) void bwd_kv_sum_kernel(BwdParams p) {
+  const int nb = p.seq / kBlk, nkb = (nb + 1) / 2, group = p.q_heads / p.kv_heads;
+  const int t = blockIdx.x & 3, kb2 = (int)(blockIdx.x >> 2) % nkb, bhk = (int)(blockIdx.x >> 2) / nkb;
+  const int n = kv_chunks(kv_items(group, nb, kb2, CAUSAL), p.chunk);
+  if (n == 1)
+    return;
+  int slot = bhk * p.per_head;  // the block's first CTA
+  if (CAUSAL) {
+    for (int k = 0; k < kb2; ++k)
+      slot += kv_chunks(kv_items(group, nb, k, true), p.chunk);
+  } else {
+    slot += kb2 * n;
+  }
+  const f32x4 *part = p.part + (size_t)slot * (16 * 512) + 4 * t * 512 + threadIdx.x;
+  f32x16 sum = {};
+  for (int c = 0; c < n; ++c) {
+    f32x4 v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      v[r] = part[(size_t)c * (16 * 512) + r * 512];
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      sum[r] += v[r >> 2][r & 3];
+  }
+  const uint32_t wave = threadIdx.x >> 6, wg = wave & 3;
+  const int role = wg & 1, dq = wg >> 1, kb = 2 * kb2 + (int)(wave >> 2);
+  if (kb >= nb)
+    return;
+  uint16_t *dst = (role ? p.dK : p.dV) + ((size_t)bhk * p.seq + (size_t)kb * kBlk) * kBD;
+  store_tile32<DT>(dst, (t >> 1) * 32, (2 * dq + (t & 1)) * 32, sum, role ? p.scale : 1.f);
 }
 
 // dQ of one 64-query block of one q head.
@@ -592,7 +539,10 @@ __global__ __launch_bounds__(256, 2) void bwd_q_kernel(BwdParams p) {
   uint8_t *sdS = smem + 2 * kKV;
   const int nb = p.seq / kBlk;
   const int pid = xcd_pid((int)blockIdx.x, (int)gridDim.x);
-  const int qb = pid % nb, bh = pid / nb;
+  const int bh = pid / nb;
+  // Causal: a head's longest query blocks first, so that the short ones fill
+  // the last round.
+  const int qb = CAUSAL ? nb - 1 - pid % nb : pid % nb;
   const int b = bh / p.q_heads, hq = bh - b * p.q_heads;
   const int hkv = hq / (p.q_heads / p.kv_heads);
   const uint32_t wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -668,23 +618,91 @@ __global__ __launch_bounds__(256, 2) void bwd_q_kernel(BwdParams p) {
 }
 
 namespace {
+// The dK/dV kernel's split: the chunk length and the CTAs a KV head then has.
+struct KvPlan {
+  int chunk = 0, per_head = 0;
+  bool sum = false;  // some block has several chunks
+};
+
+// A CTA takes 1.75 us an item (measured) and 4 to start and end; a CU runs one
+// at a time.  Splitting adds the sum kernel: 4 us and 0.06 a CTA (its 128 KiB
+// partial written and read).  Whole blocks on n > CUs: the CUs share the total,
+// and the last blocks run up to half a block's time alone.  Candidates: whole
+// blocks, or the shortest chunks for which the CTAs fill the chip once, twice
+// or three times.  B2 Hq16 Hkv4 S2048 causal (128 blocks of 8 to 128 items):
+// whole 229 us, chunks of 43 items (256 CTAs) 105 to 111 and the sum 7.5.  S1984
+// (a half block at the end): the backward 346 -> 196 us, against 64-key blocks of
+// one CTA each.
+KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, int cus) {
+  const int64_t heads = (int64_t)batch * kv_heads;
+  const int nkb = (nb + 1) / 2, longest = group * nb;
+  auto per_head = [&](int chunk) {
+    if (!causal)
+      return (int64_t)nkb * kv_chunks(longest, chunk);
+    int64_t n = 0;
+    for (int k = 0; k < nkb; ++k)
+      n += kv_chunks(kv_items(group, nb, k, true), chunk);
+    return n;
+  };
+  int64_t total = 0;  // items of a head
+  for (int k = 0; k < nkb; ++k)
+    total += kv_items(group, nb, k, causal);
+  auto time = [&](int64_t ctas, int len) {
+    const double share = (double)total * heads / cus;
+    return 4 + 1.75 * (ctas <= cus ? (double)len : share + 0.5 * len + 2);
+  };
+  KvPlan plan;
+  plan.per_head = nkb;
+  double best = time(heads * nkb, longest);
+  for (int rounds = 1; rounds <= 3; ++rounds) {
+    const int64_t most = (int64_t)rounds * cus / heads;
+    if (most <= nkb)
+      continue;
+    int lo = 1, hi = longest;  // the least chunk with per_head(chunk) <= most
+    while (lo < hi) {
+      const int mid = (lo + hi) / 2;
+      if (per_head(mid) <= most)
+        hi = mid;
+      else
+        lo = mid + 1;
+    }
+    const int64_t n = per_head(lo);
+    if (lo == longest || n == nkb)
+      continue;
+    const double t = time(heads * n, lo) + 4 + 0.06 * (double)(heads * n);
+    if (t < best) {
+      best = t;
+      plan.chunk = lo;
+      plan.per_head = (int)n;
+      plan.sum = true;
+    }
+  }
+  return plan;
+}
+
+constexpr size_t kPartBytes = 16 * 512 * sizeof(f32x4);  // a CTA's dK, dV in fp32
+
 template <int DT, bool CAUSAL>
-hipError_t launch_bwd_dt(const BwdParams &p, hipStream_t stream) {
+hipError_t launch_bwd_dt(const BwdParams &p, bool sum, hipStream_t stream) {
   const int rows = p.batch * p.q_heads * p.seq;
   hipLaunchKernelGGL((bwd_delta_kernel<DT>), dim3((rows + 15) / 16), dim3(256), 0, stream, p,
                      rows);
-  const int nb = p.seq / kBlk;
-  if (nb % 2 == 0)
-    hipLaunchKernelGGL((bwd_kv_pp_kernel<DT, CAUSAL>), dim3(nb / 2 * p.batch * p.kv_heads),
-                       dim3(512), 0, stream, p);
-  else
-    hipLaunchKernelGGL((bwd_kv_kernel<DT, CAUSAL>), dim3(nb * p.batch * p.kv_heads), dim3(256),
+  const int nb = p.seq / kBlk, heads = p.batch * p.kv_heads;
+  hipLaunchKernelGGL((bwd_kv_pp_kernel<DT, CAUSAL>), dim3(p.per_head * heads), dim3(512), 0, stream,
+                     p);
+  if (sum)
+    hipLaunchKernelGGL((bwd_kv_sum_kernel<DT, CAUSAL>), dim3((nb + 1) / 2 * heads * 4), dim3(512),
                        0, stream, p);
   hipLaunchKernelGGL((bwd_q_kernel<DT, CAUSAL>), dim3(nb * p.batch * p.q_heads), dim3(256), 0,
                      stream, p);
   return hipGetLastError();
 }
 } // namespace
+
+size_t bwd_workspace_bytes(int batch, int q_heads, int kv_heads, int seq, bool causal, int cus) {
+  const KvPlan plan = kv_plan(batch, kv_heads, q_heads / kv_heads, seq / kBlk, causal, cus);
+  return plan.sum ? (size_t)batch * kv_heads * plan.per_head * kPartBytes : 0;
+}
 
 hipError_t launch_bwd(const BwdArgs &a, hipStream_t stream) {
   BwdParams p{};
@@ -706,9 +724,21 @@ hipError_t launch_bwd(const BwdArgs &a, hipStream_t stream) {
   p.scale = a.scale > 0.f ? a.scale : 1.0f / __builtin_sqrtf((float)kBD);
   p.scale_log2 = p.scale * kLog2eB;
   p.inv_scale = 1.0f / p.scale;
+  KvPlan plan = kv_plan(a.batch, a.kv_heads, a.q_heads / a.kv_heads, a.seq / kBlk, a.causal != 0,
+                        a.cus);
+  if (plan.sum && (!a.workspace || a.workspace_bytes < (size_t)a.batch * a.kv_heads *
+                                                           plan.per_head * kPartBytes)) {
+    plan = KvPlan{};
+    plan.per_head = (a.seq / kBlk + 1) / 2;
+  }
+  p.chunk = plan.chunk;
+  p.per_head = plan.per_head;
+  p.part = static_cast<f32x4 *>(a.workspace);
   if (a.dtype == kF16)
-    return a.causal ? launch_bwd_dt<kF16, true>(p, stream) : launch_bwd_dt<kF16, false>(p, stream);
-  return a.causal ? launch_bwd_dt<kBF16, true>(p, stream) : launch_bwd_dt<kBF16, false>(p, stream);
+    return a.causal ? launch_bwd_dt<kF16, true>(p, plan.sum, stream)
+                    : launch_bwd_dt<kF16, false>(p, plan.sum, stream);
+  return a.causal ? launch_bwd_dt<kBF16, true>(p, plan.sum, stream)
+                  : launch_bwd_dt<kBF16, false>(p, plan.sum, stream);
 }
 
 } // namespace attention

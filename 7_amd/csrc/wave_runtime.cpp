@@ -672,6 +672,36 @@ int wave_fa_bwd_launch(const void *Q, const void *K, const void *V, const void *
                        const void *dO, const float *lse, float *delta, void *dQ, void *dK,
                        void *dV, int batch, int q_heads, int kv_heads, int seq, int head_dim,
                        int dtype, int causal, float scale, void *stream) {
+  return wave_fa_bwd_workspace_launch(Q, K, V, O, dO, lse, delta, dQ, dK, dV, batch, q_heads,
+                                      kv_heads, seq, head_dim, dtype, causal, scale, nullptr, 0,
+                                      stream);
+}
+
+int wave_fa_bwd_workspace_bytes(int batch, int q_heads, int kv_heads, int seq, int causal,
+                                size_t *bytes) {
+  if (!bytes)
+    return fail(WAVE_ERR_INVALID, "fa_bwd: null size output");
+  if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || seq <= 0 || q_heads % kv_heads != 0)
+    return fail(WAVE_ERR_INVALID, "fa_bwd: batch=%d q_heads=%d kv_heads=%d seq=%d", batch, q_heads,
+                kv_heads, seq);
+  if (causal != 0 && causal != 1)
+    return fail(WAVE_ERR_INVALID, "fa_bwd: causal=%d must be 0 or 1", causal);
+  if (seq % 64 != 0 || (int64_t)batch * q_heads * seq > INT32_MAX / 2)
+    return fail(WAVE_ERR_UNSUPPORTED, "fa_bwd: seq=%d must be a multiple of 64, the problem "
+                "below 2^30 rows", seq);
+  int cus = 0;
+  const int st = device_cus(&cus);
+  if (st != WAVE_OK)
+    return st;
+  *bytes = wave::attention::bwd_workspace_bytes(batch, q_heads, kv_heads, seq, causal != 0, cus);
+  return WAVE_OK;
+}
+
+int wave_fa_bwd_workspace_launch(const void *Q, const void *K, const void *V, const void *O,
+                                 const void *dO, const float *lse, float *delta, void *dQ,
+                                 void *dK, void *dV, int batch, int q_heads, int kv_heads,
+                                 int seq, int head_dim, int dtype, int causal, float scale,
+                                 void *workspace, size_t workspace_bytes, void *stream) {
   if (!Q || !K || !V || !O || !dO || !lse || !delta || !dQ || !dK || !dV)
     return fail(WAVE_ERR_INVALID, "fa_bwd: null pointer argument");
   if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || seq <= 0)
@@ -717,6 +747,13 @@ int wave_fa_bwd_launch(const void *Q, const void *K, const void *V, const void *
   a.dtype = dtype;
   a.causal = causal;
   a.scale = scale;
+  a.workspace = workspace;
+  a.workspace_bytes = workspace_bytes;
+  if ((uintptr_t)workspace & 15)
+    return fail(WAVE_ERR_INVALID, "fa_bwd: workspace must be 16-byte aligned");
+  const int st = device_cus(&a.cus);
+  if (st != WAVE_OK)
+    return st;
   return hip_status(wave::attention::launch_bwd(a, static_cast<hipStream_t>(stream)),
                     "wave_fa_bwd_launch");
 }

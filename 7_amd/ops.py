@@ -384,7 +384,7 @@ def flash_attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: to
                         scale: float | None = None
                         ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """dQ, dK, dV of O = softmax(scale Q K^T) V given dO, O and the forward's
-    lse (flash_attention_lse); wave_fa_bwd_launch.  seq % 64 == 0."""
+    lse (flash_attention_lse); wave_fa_bwd_workspace_launch.  seq % 64 == 0."""
     B, Hq, Hkv, S, D = _fa_shapes(q, k, v)
     for t, n in ((o, "o"), (do, "do")):
         _need(t, n, q.device)
@@ -395,10 +395,17 @@ def flash_attention_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: to
         raise ValueError("lse must be float32 [batch, q_heads, seq]")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     delta = torch.empty((B, Hq, S), dtype=torch.float32, device=q.device)
-    rt.check(rt.lib().wave_fa_bwd_launch(
+    # The dK/dV work split's partials, for sizes the launch takes at all.
+    need = ctypes.c_size_t()
+    if B > 0 and Hkv > 0 and Hq % Hkv == 0 and S > 0 and S % 64 == 0:
+        rt.check(rt.lib().wave_fa_bwd_workspace_bytes(B, Hq, Hkv, S, int(causal),
+                                                      ctypes.byref(need)))
+    ws = torch.empty(need.value, dtype=torch.uint8, device=q.device) if need.value else None
+    rt.check(rt.lib().wave_fa_bwd_workspace_launch(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(), lse.data_ptr(),
         delta.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, Hq, Hkv, S, D,
-        _DT[q.dtype], int(causal), float(scale or 0.0), _stream(q)))
+        _DT[q.dtype], int(causal), float(scale or 0.0),
+        ws.data_ptr() if ws is not None else None, need.value, _stream(q)))
     return dq, dk, dv
 
 

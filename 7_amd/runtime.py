@@ -49,6 +49,8 @@ _SIGNATURES = {
     "wave_fa_fwd_mxfp8_launch": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I,
                                       _I, _F, _P]),
     "wave_mxfp8_quantize_launch": (_I, [_P, _P, _P, _L, _L, _L, _I, _P]),
+    "wave_fa_bwd_workspace_bytes": (_I, [_I, _I, _I, _I, _I, ctypes.POINTER(_SZ)]),
+    "wave_fa_bwd_workspace_launch": (_I, [_P] * 10 + [_I] * 7 + [_F, _P, _SZ, _P]),
     "wave_fa_bwd_launch": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I,
                                 _I, _I, _F, _P]),
     "wave_status_string": (ctypes.c_char_p, [_I]),

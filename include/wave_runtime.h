@@ -300,6 +300,19 @@ int wave_fa_bwd_launch(const void *Q, const void *K, const void *V, const void *
                        void *dV, int batch, int q_heads, int kv_heads, int seq, int head_dim,
                        int dtype, int causal, float scale, void *stream);
 
+/* The same with a workspace (caller-owned, 16-byte aligned, any contents, one
+ * launch in flight), which lets the dK/dV kernel cut its key blocks' work into
+ * chunks for several CTAs where the blocks are fewer than the CUs or causal
+ * ones of uneven length; wave_fa_bwd_workspace_bytes gives its size (0 where
+ * whole blocks are used).  A smaller one (or none) runs whole blocks. */
+int wave_fa_bwd_workspace_bytes(int batch, int q_heads, int kv_heads, int seq, int causal,
+                                size_t *bytes);
+int wave_fa_bwd_workspace_launch(const void *Q, const void *K, const void *V, const void *O,
+                                 const void *dO, const float *lse, float *delta, void *dQ,
+                                 void *dK, void *dV, int batch, int q_heads, int kv_heads,
+                                 int seq, int head_dim, int dtype, int causal, float scale,
+                                 void *workspace, size_t workspace_bytes, void *stream);
+
 /* ---- flash_attention_f32 ------------------------------------------------
  * Replaces `flash_attention_f32(Q, K, V, O)` (wave_attention.py:1406-1441;
  * wave-fa-calibrate-runner.cpp:346-361): Q [block_m][head_dim] f16

@@ -128,3 +128,43 @@ def test_fa_bwd_rejects_ragged_seq(wave, dev):
     lse = torch.zeros((1, 1, 100), dtype=torch.float32, device=dev)
     with pytest.raises(NotImplementedError, match="multiple of 64"):
         wave.flash_attention_bwd(t, t, t, t, t, lse)
+
+
+# Shapes whose key blocks are cut into chunks for several CTAs (fewer blocks
+# than CUs, or causal ones of uneven length), with whole blocks left uncut, an
+# odd number of 64-key blocks (the last 128-key block half past the sequence)
+# and one head; every gradient against the launch without a workspace (one CTA
+# a block): the sums differ in order only, so by fp32 rounding before the one
+# rounding to dtype (at most one unit in the last place of a few elements).
+@pytest.mark.parametrize("dt", [1, 2])
+@pytest.mark.parametrize("B,Hq,Hkv,S,causal", [(1, 4, 1, 64, False), (1, 8, 2, 448, True),
+                                                (2, 4, 2, 1024, True), (1, 1, 1, 1984, False),
+                                                (1, 6, 2, 832, False), (1, 16, 2, 2048, True)])
+def test_fa_bwd_work_split(wave, dev, dt, B, Hq, Hkv, S, causal):
+    import ctypes
+
+    rt = wave.runtime
+    need = ctypes.c_size_t()
+    rt.check(rt.lib().wave_fa_bwd_workspace_bytes(B, Hq, Hkv, S, int(causal), ctypes.byref(need)))
+    if torch.cuda.get_device_properties(dev).multi_processor_count == 256:
+        assert need.value > 0
+    g = torch.Generator().manual_seed(31)
+    q, k, v, do = (torch.randn(s, generator=g).to(TDT[dt]).to(dev)
+                   for s in ((B, Hq, S, 128), (B, Hkv, S, 128), (B, Hkv, S, 128), (B, Hq, S, 128)))
+    o, lse = wave.flash_attention_lse(q, k, v, causal=causal)
+    got = wave.flash_attention_bwd(q, k, v, o, do, lse, causal=causal)
+    again = wave.flash_attention_bwd(q, k, v, o, do, lse, causal=causal)
+    want = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+    delta = torch.empty_like(lse)
+    st = torch.cuda.current_stream().cuda_stream
+    rt.check(rt.lib().wave_fa_bwd_launch(
+        *(t.data_ptr() for t in (q, k, v, o, do, lse, delta, *want)), B, Hq, Hkv, S, 128, dt,
+        int(causal), 0.0, st))
+    torch.cuda.synchronize()
+    ulp = {1: 2.0 ** -10, 2: 2.0 ** -7}[dt]
+    for name, x, x2, y in zip(("dq", "dk", "dv"), got, again, want):
+        assert torch.equal(x, x2), f"{name} differs from run to run"
+        d = (x.double() - y.double()).abs()
+        bound = ulp * y.double().abs() + 1e-5 * y.double().abs().max()
+        assert bool((d <= bound).all()), f"{name}: {d.max().item()}"
+        assert (d > 0).double().mean().item() < 0.05, f"{name}: {(d > 0).double().mean().item()}"

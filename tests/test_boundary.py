@@ -390,3 +390,17 @@ def test_mxfp8_quantize_rejects_bad_arguments(wave, kw, status):
     st = L.wave_mxfp8_quantize_launch(a["X"], a["E"], a["S"], a["outer"], a["n"], a["inner"],
                                       a["dt"], None)
     assert st == status and L.wave_last_error()
+
+
+@pytest.mark.parametrize("kw,status", [
+    (dict(batch=0), -1), (dict(q_heads=3, kv_heads=2), -1), (dict(causal=2), -1),
+    (dict(seq=100), -2), (dict(seq=1 << 30), -2), (dict(out=False), -1),
+])
+def test_fa_bwd_workspace_rejects_bad_arguments(wave, kw, status):
+    L = wave.runtime.lib()
+    a = dict(batch=1, q_heads=2, kv_heads=2, seq=128, causal=0, out=True)
+    a.update(kw)
+    n = ctypes.c_size_t()
+    st = L.wave_fa_bwd_workspace_bytes(a["batch"], a["q_heads"], a["kv_heads"], a["seq"],
+                                       a["causal"], ctypes.byref(n) if a["out"] else None)
+    assert st == status and L.wave_last_error()
