@@ -22,7 +22,22 @@ hipError_t launch_fwd(const FwdArgs &a, hipStream_t stream) {
   p.kv_heads = a.kv_heads;
   p.seq_q = a.seq_q;
   p.seq_k = a.seq_k;
-  const int rows = a.waves == kR3Waves ? kR3Rows : 32 * kPPWaves;  // 4 waves: 256 too
+  // The default (8 waves a 256-row block, one CTA a CU) gives way to the 4-wave
+  // kernel on 128-row blocks where those are at most one a CU (half as many
+  // 256-row ones would leave CUs idle: B1 Hq32 Hkv8 S1000 causal bf16 32.7 -> 26.0
+  // us, B1 H8 S512 16.8 -> 13.0, B1 H16 S1024 28.8 -> 23.1; at 384 blocks of 128
+  // the 8-wave kernel is ahead, 24.8 / 28.0), or where, on more than one
+  // round of 256-row blocks, they save more padded rows than their rate costs
+  // (about 13 % behind on a full chip: B8 H64 S300 57.9 -> 43.3, B7 H11 S777
+  // causal 54.1 -> 34.4, S1024 level; within one round the 8-wave kernel keeps
+  // ahead, B1 H61 S640 24.3 / 25.7).
+  const int64_t heads = (int64_t)a.batch * a.q_heads;
+  const int64_t n128 = ((a.seq_q - 1) / kF4PassRows + 1) * heads,
+                n256 = ((a.seq_q - 1) / 256 + 1) * heads;
+  const bool narrow = a.waves == kPPWaves && (n128 <= a.cus || (n256 > a.cus && 113 * n128 < 200 * n256));
+  const int rows = a.waves == kR3Waves ? kR3Rows
+                   : narrow            ? kF4PassRows
+                                       : 32 * kPPWaves;  // 4 waves: two passes of 128
   p.q_blocks = (a.seq_q + rows - 1) / rows;
   p.causal = a.causal;
   const float scale = a.scale > 0.f ? a.scale : 1.0f / std::sqrt((float)a.head_dim);
@@ -32,20 +47,22 @@ hipError_t launch_fwd(const FwdArgs &a, hipStream_t stream) {
   // units (wave_flash_attention.py:108-113 with scale = 1/sqrt(128)).
   p.fixed_max = (float)((double)kLog2e * scale * a.head_dim * a.qk_max_abs * a.qk_max_abs);
   const bool fixed = a.qk_max_abs > 0.f;
-  if (a.waves == kF4Waves) {
-    // 4 waves x 64 query rows per CTA (the same 256-row blocks).
+  if (a.waves == kF4Waves || narrow) {
+    // 4 waves x 32 query rows per pass, two passes a CTA (the same 256-row
+    // blocks) or one.
     const dim3 grid(p.q_blocks * a.batch * a.q_heads), block(64 * kF4Waves);
-    if (a.dtype == kF16) {
-      if (fixed)
-        hipLaunchKernelGGL((fwd4_kernel<kF16, true>), grid, block, 0, stream, p);
+    auto go = [&](auto dt, auto fix) {
+      constexpr int DT = decltype(dt)::value;
+      constexpr bool FIXED = decltype(fix)::value;
+      if (narrow)
+        hipLaunchKernelGGL((fwd4_kernel<DT, FIXED, 1>), grid, block, 0, stream, p);
       else
-        hipLaunchKernelGGL((fwd4_kernel<kF16, false>), grid, block, 0, stream, p);
-    } else {
-      if (fixed)
-        hipLaunchKernelGGL((fwd4_kernel<kBF16, true>), grid, block, 0, stream, p);
-      else
-        hipLaunchKernelGGL((fwd4_kernel<kBF16, false>), grid, block, 0, stream, p);
-    }
+        hipLaunchKernelGGL((fwd4_kernel<DT, FIXED, 2>), grid, block, 0, stream, p);
+    };
+    if (a.dtype == kF16)
+      fixed ? go(I_<kF16>{}, std::true_type{}) : go(I_<kF16>{}, std::false_type{});
+    else
+      fixed ? go(I_<kBF16>{}, std::true_type{}) : go(I_<kBF16>{}, std::false_type{});
     return hipGetLastError();
   }
   if (a.waves == kR3Waves) {

@@ -11,7 +11,8 @@
 // (log2 units), v_dot2 row sums of the packed P, optional fixed max.  The
 // schedule differs:
 //  * 4 waves x 32 query rows = 128 rows per pass; a CTA runs its 256 rows
-//    as two passes over the keys.  64 KiB of LDS and at most 256 VGPRs let
+//    as two passes over the keys (or 128 rows as one: the library's forward
+//    of small grids).  64 KiB of LDS and at most 256 VGPRs let
 //    two CTAs share a CU, so each SIMD holds two waves of different CTAs
 //    whose MFMA and softmax work overlap.
 //  * Within a wave, a two-phase pipeline per 64-key tile: phase 1 issues
@@ -42,9 +43,9 @@ constexpr int kVt4Bytes = kD * kVt4Pitch;        // 17 KiB
 constexpr int kF4Smem = 2 * kKBytes + 2 * kVt4Bytes;
 
 // CTA `raw` of a grid of q_blocks * batch * q_heads CTAs of 256 threads
-// (q_blocks = ceil(seq_q / 256)).  smem: kF4Smem bytes of 1024-byte-aligned
-// LDS.  FIXED as in fwd_pp_cta.
-template <int DT, bool FIXED = false>
+// (q_blocks = ceil(seq_q / (128 PASSES))).  smem: kF4Smem bytes of
+// 1024-byte-aligned LDS.  FIXED as in fwd_pp_cta.
+template <int DT, bool FIXED = false, int PASSES = 2>
 __device__ __forceinline__ void fwd4_cta(const Params &p, int raw, uint8_t *smem) {
   int bh, qb;
   block_coords(p, raw, bh, qb);
@@ -61,8 +62,8 @@ __device__ __forceinline__ void fwd4_cta(const Params &p, int raw, uint8_t *smem
   auto pin = [](auto x) { asm volatile("" ::"v"(x)); };
 
 #pragma unroll 1
-  for (int pass = 0; pass < 2; ++pass) {
-    const int q0 = qb * (2 * kF4PassRows) + pass * kF4PassRows;
+  for (int pass = 0; pass < PASSES; ++pass) {
+    const int q0 = qb * (PASSES * kF4PassRows) + pass * kF4PassRows;
     if (q0 >= p.seq_q)
       break;
     // Per-lane values are derived inside the pass (from a thread id the
@@ -377,10 +378,10 @@ __device__ __forceinline__ void fwd4_cta(const Params &p, int raw, uint8_t *smem
   }
 }
 
-template <int DT, bool FIXED>
+template <int DT, bool FIXED, int PASSES>
 __global__ __launch_bounds__(64 * kF4Waves, 2) void fwd4_kernel(Params p) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kF4Smem];
-  fwd4_cta<DT, FIXED>(p, blockIdx.x, smem);
+  fwd4_cta<DT, FIXED, PASSES>(p, blockIdx.x, smem);
 }
 
 } // namespace attention

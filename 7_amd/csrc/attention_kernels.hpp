@@ -71,10 +71,10 @@ struct Params {
 // Linear CTA id -> (batch*head, query block).
 __device__ __forceinline__ void block_coords(const Params &p, int raw, int &bh, int &qb) {
   const int total = p.q_blocks * p.batch * p.q_heads;
-  // Dispatch puts CTA i on XCD i % 8; make consecutive pids share an XCD.
-  int pid = raw;
-  if ((total & 7) == 0)
-    pid = (raw & 7) * (total >> 3) + (raw >> 3);
+  // Dispatch puts CTA i on XCD i % 8; make consecutive pids share an XCD (the
+  // first total % 8 XCDs hold one more).
+  const int xcd = raw & 7;
+  const int pid = xcd * (total >> 3) + min(xcd, total & 7) + (raw >> 3);
   bh = pid / p.q_blocks;
   qb = pid - bh * p.q_blocks;
   if (p.causal)

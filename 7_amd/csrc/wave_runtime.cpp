@@ -653,6 +653,9 @@ int fa_fwd(const void *Q, const void *K, const void *V, void *O, int batch, int 
   a.qk_max_abs = qk_max_abs;
   a.waves = waves;
   a.lse = lse;
+  const int st = device_cus(&a.cus);
+  if (st != WAVE_OK)
+    return st;
   return hip_status(wave::attention::launch_fwd(a, static_cast<hipStream_t>(stream)), name);
 }
 } // namespace
