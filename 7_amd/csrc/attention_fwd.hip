@@ -6,6 +6,7 @@
 #include "attention_fwd4.hpp"
 #include "attention_kernels.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace wave {
@@ -31,10 +32,26 @@ hipError_t launch_fwd(const FwdArgs &a, hipStream_t stream) {
   // (about 13 % behind on a full chip: B8 H64 S300 57.9 -> 43.3, B7 H11 S777
   // causal 54.1 -> 34.4, S1024 level; within one round the 8-wave kernel keeps
   // ahead, B1 H61 S640 24.3 / 25.7).
+  // Causal blocks are of uneven length: where the heads divide over the XCDs they
+  // go by length (block_coords).  8-wave kernel, head by head -> by length:
+  // B4 Hq32 Hkv32 S3000 107 -> 84 us (B1), B4 H16 S2048 104 -> 78, B2 Hq32 Hkv8
+  // S4096 309 -> 277, B1 Hq64 Hkv8 S8192 1013 -> 979.  The heads then side by
+  // side read their K and V at once, which the 256 MB last-level cache has to
+  // hold: 32 MB in all (B1 Hq32 Hkv4 S16384) 1965 -> 1937 us, 256 MB (B4 H32
+  // S4096, B8 H32 S2048) 623 -> 587 and 383 -> 351, 512 MB (B2 H64 S8192) 2063 ->
+  // 2228.  In long and short pairs the 4-wave kernel's blocks are ahead up to two
+  // of them a CU: B2 Hq16 Hkv4 S2048 59 (8-wave, head by head), 53 (8-wave, by
+  // length), 47 (pairs); B1 H16 S4096 103, 98, 91; with four a CU B1 Hq64 Hkv8
+  // S2048 114, 77, 82.  One block a CU has nothing to order (B1 Hq32 Hkv8 S1000
+  // 23.4 head by head, 24.1 by length).
   const int64_t heads = (int64_t)a.batch * a.q_heads;
   const int64_t n128 = ((a.seq_q - 1) / kF4PassRows + 1) * heads,
                 n256 = ((a.seq_q - 1) / 256 + 1) * heads;
-  const bool narrow = a.waves == kPPWaves && (n128 <= a.cus || (n256 > a.cus && 113 * n128 < 200 * n256));
+  const bool by_length = a.causal && heads % 8 == 0 &&
+                         (int64_t)a.batch * a.kv_heads * a.seq_k * (2 * kKRowBytes) <= (256 << 20);
+  const bool narrow = a.waves == kPPWaves && (n128 <= (by_length ? 2 * a.cus : a.cus) ||
+                                              (n256 > a.cus && 113 * n128 < 200 * n256));
+  p.by_length = !by_length ? 0 : !narrow ? 1 : n128 > a.cus ? std::max(a.cus / 8, 1) : 0;
   const int rows = a.waves == kR3Waves ? kR3Rows
                    : narrow            ? kF4PassRows
                                        : 32 * kPPWaves;  // 4 waves: two passes of 128

@@ -66,14 +66,31 @@ struct Params {
   float scale_log2;  // softmax scale * log2(e)
   float fixed_max;   // fixed-max kernels: the row max of every row (log2 units)
   float *lse;        // optional [batch*q_heads][seq_q]: ln sum_k exp(scale * q.k)
+  int by_length;     // CTA order (block_coords); > 0 only causal, q_heads * batch % 8 == 0
 };
 
-// Linear CTA id -> (batch*head, query block).
+// Linear CTA id -> (batch*head, query block).  Dispatch puts CTA i on XCD
+// i % 8; the CTAs of one head share an XCD (its K and V stay in that L2), causal
+// ones with the longest query blocks first.  by_length > 0: an XCD runs the
+// longest blocks of all its heads first, then the next, so that the last CTAs to
+// start are the shortest of all.  by_length = n > 1: of an XCD's CTAs every
+// second run of n (one for each of its CUs) is reversed; where two CTAs share a
+// CU these are then a long and a short one, and the CUs' sums are alike.
 __device__ __forceinline__ void block_coords(const Params &p, int raw, int &bh, int &qb) {
-  const int total = p.q_blocks * p.batch * p.q_heads;
-  // Dispatch puts CTA i on XCD i % 8; make consecutive pids share an XCD (the
-  // first total % 8 XCDs hold one more).
+  const int heads = p.batch * p.q_heads, total = p.q_blocks * heads;
   const int xcd = raw & 7;
+  if (p.by_length > 0) {
+    const int hx = heads >> 3;  // heads of an XCD
+    int i = raw >> 3;
+    if (p.by_length > 1 && (i / p.by_length) & 1) {
+      const int lo = i / p.by_length * p.by_length, hi = min(lo + p.by_length, hx * p.q_blocks);
+      i = lo + (hi - 1 - i);
+    }
+    bh = xcd * hx + i % hx;
+    qb = p.q_blocks - 1 - i / hx;
+    return;
+  }
+  // The first total % 8 XCDs hold one CTA more.
   const int pid = xcd * (total >> 3) + min(xcd, total & 7) + (raw >> 3);
   bh = pid / p.q_blocks;
   qb = pid - bh * p.q_blocks;

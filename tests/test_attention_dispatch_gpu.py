@@ -59,3 +59,14 @@ def test_every_row(wave, dev, dt, causal, B, Hq, Hkv, S):
         rb, _ = reference(qb, kb, v, causal)
         over = ((ob.double() - rb).abs() - half_ulp * rb.abs()).max().item()
         assert over <= TOL[dt], over
+
+
+# Causal blocks by length (heads a multiple of the 8 XCDs): long and short pairs
+# of 128-row blocks (1100 and 2300: a last run of blocks that is not full; 300;
+# 257: four blocks a CU, mostly padding) and 256-row blocks (1537, 777), odd
+# lengths throughout, K and V of one head up to all of them.
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,S", [(1, 32, 8, 1100), (2, 8, 1, 2300), (2, 72, 8, 300),
+                                         (8, 40, 8, 257), (1, 40, 40, 1537), (4, 24, 8, 777)])
+def test_blocks_by_length(wave, dev, dt, B, Hq, Hkv, S):
+    test_every_row(wave, dev, dt, True, B, Hq, Hkv, S)
