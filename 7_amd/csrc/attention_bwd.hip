@@ -40,6 +40,8 @@
 #include "attention.hpp"
 #include "wave_common.hpp"
 
+#include <algorithm>
+
 namespace wave {
 namespace attention {
 
@@ -80,6 +82,8 @@ struct BwdParams {
   // `per_head` CTAs a KV head, partials [CTA][16][512] f32x4.
   int chunk, per_head;
   f32x4 *part;
+  // Causal CTA order (head_coords) of the dK/dV and the dQ kernel.
+  int kv_by_length, q_by_length;
 };
 
 // Two NT products over K = 128 that share their A rows: c0 += A0 . b0^T and
@@ -225,6 +229,21 @@ __device__ __forceinline__ int xcd_pid(int raw, int total) {
   return xcd * (total >> 3) + min(xcd, total & 7) + (raw >> 3);
 }
 
+// CTA id -> head and the head's CTA i of n; by_length (heads a multiple of 8):
+// an XCD runs CTA 0 of each of its heads, then CTA 1 of each, and so on.
+__device__ __forceinline__ void head_coords(int raw, int heads, int n, int by_length, int &head,
+                                            int &i) {
+  if (by_length) {
+    const int hx = heads >> 3, j = raw >> 3;  // heads of an XCD
+    i = j / hx;
+    head = (raw & 7) * hx + j - i * hx;
+    return;
+  }
+  const int pid = xcd_pid(raw, heads * n);
+  head = pid / n;
+  i = pid - head * n;
+}
+
 // Store a 32x32 fp32 accumulator tile (rows row0.., columns col0..) of a
 // [rows][128] 16-bit output, times mul.
 template <int DT>
@@ -329,13 +348,13 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
   constexpr uint32_t kStats = 2 * kWide, kQD = kStats + 512;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[3 * kQD + 4 * kNarrowS];
   const int nb = p.seq / kBlk;
-  const int pid = xcd_pid((int)blockIdx.x, (int)gridDim.x);
-  const int bhk = pid / p.per_head;
+  int bhk, cta;
+  head_coords((int)blockIdx.x, p.batch * p.kv_heads, p.per_head, p.kv_by_length, bhk, cta);
   const int b = bhk / p.kv_heads, hkv = bhk - b * p.kv_heads;
   const int group = p.q_heads / p.kv_heads;
   const uint32_t wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const uint32_t grp = wave >> 2, wg = wave & 3;
-  const KvChunk chunk = kv_chunk<CAUSAL>(p, group, nb, pid - bhk * p.per_head);
+  const KvChunk chunk = kv_chunk<CAUSAL>(p, group, nb, cta);
   const int kb2 = chunk.kb2;
   // This group's 64-key block; past the sequence (the last block's second half
   // when nb is odd) it repeats the last one and stores nothing.
@@ -344,9 +363,9 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
   const size_t kv_off = ((size_t)bhk * p.seq + (size_t)kb * kBlk) * kBD;
   uint8_t *sPt = smem + 3 * kQD + grp * 2 * kNarrowS, *sdSt = sPt + kNarrowS;
   const uint32_t lds0 = lds_addr(smem);
-  // Wave roles within the group.  Score products: query half qh2, key half kh2.  Gradient products: wave
-  // role 0 accumulates dV, role 1 dK, each for all 64 keys of the group and
-  // d columns 64 dq .. 64 dq + 63.
+  // Wave roles within the group.  Score products: query half qh2, key half
+  // kh2.  Gradient products: wave role 0 accumulates dV, role 1 dK, each for
+  // all 64 keys of the group and d columns 64 dq .. 64 dq + 63.
   const int qh2 = wg & 1, kh2 = wg >> 1, role = wg & 1, dq = wg >> 1;
   u32x4 kf[8], vf[8];
   load_frags(p.K + kv_off + (size_t)(kh2 * 32 + (lane & 31)) * kBD, kf);
@@ -405,11 +424,17 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
       }
     }
   };
-  Cursor dmac{first / (nb - qb0), qb0 + first % (nb - qb0)}, cur = dmac;
+  const int h0 = first / (nb - qb0);
+  Cursor dmac{h0, qb0 + first - h0 * (nb - qb0)}, cur = dmac;
   if (grp == 1)
     dma_item(dmac, 0);
   advance(dmac);
   vm_wait_barrier();
+  // Waited for here: a kernel argument still on its way counts as an LDS read to
+  // the compiler, which then drains all reads at each fragment's wait in the loop
+  // (B1 Hq64 Hkv8 S8192 7.39 ms, 7.65 without).
+  f32x4 *part0 = p.part;
+  asm volatile("" : "+s"(part0));
   const int nseg = 2 * items + 2;
   for (int sg = 0; sg < nseg; ++sg) {
     if ((sg & 1) == 0 && (sg >> 1) + 1 < items) {
@@ -465,7 +490,7 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
       lds_barrier();
   }
   if (chunk.count > 1) {
-    f32x4 *part = p.part + (size_t)pid * (16 * 512) + threadIdx.x;
+    f32x4 *part = part0 + (size_t)(bhk * p.per_head + cta) * (16 * 512) + threadIdx.x;
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -538,11 +563,11 @@ __global__ __launch_bounds__(256, 2) void bwd_q_kernel(BwdParams p) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * kKV + kNarrowS];
   uint8_t *sdS = smem + 2 * kKV;
   const int nb = p.seq / kBlk;
-  const int pid = xcd_pid((int)blockIdx.x, (int)gridDim.x);
-  const int bh = pid / nb;
-  // Causal: a head's longest query blocks first, so that the short ones fill
-  // the last round.
-  const int qb = CAUSAL ? nb - 1 - pid % nb : pid % nb;
+  // Causal: the longest query blocks first, so that the short ones fill the
+  // last round.
+  int bh, i;
+  head_coords((int)blockIdx.x, p.batch * p.q_heads, nb, p.q_by_length, bh, i);
+  const int qb = CAUSAL ? nb - 1 - i : i;
   const int b = bh / p.q_heads, hq = bh - b * p.q_heads;
   const int hkv = hq / (p.q_heads / p.kv_heads);
   const uint32_t wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -627,13 +652,16 @@ struct KvPlan {
 // A CTA takes 1.75 us an item (measured) and 4 to start and end; a CU runs one
 // at a time.  Splitting adds the sum kernel: 4 us and 0.06 a CTA (its 128 KiB
 // partial written and read).  Whole blocks on n > CUs: the CUs share the total,
-// and the last blocks run up to half a block's time alone.  Candidates: whole
-// blocks, or the shortest chunks for which the CTAs fill the chip once, twice
-// or three times.  B2 Hq16 Hkv4 S2048 causal (128 blocks of 8 to 128 items):
-// whole 229 us, chunks of 43 items (256 CTAs) 105 to 111 and the sum 7.5.  S1984
-// (a half block at the end): the backward 346 -> 196 us, against 64-key blocks of
-// one CTA each.
-KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, int cus) {
+// and the last blocks run up to half a block's time alone; causal ones by length
+// end with the shortest, and their time is the total's share or the longest.
+// Candidates: whole blocks, or the shortest chunks for which the CTAs fill the
+// chip once, twice or three times.  B2 Hq16 Hkv4 S2048 causal (128 blocks of 8 to
+// 128 items): whole 229 us, chunks of 43 items (256 CTAs) 105 to 111 and the sum
+// 7.5.  S1984 (a half block at the end): the backward 346 -> 196 us, against 64-key
+// blocks of one CTA each.  B2 Hq32 Hkv8 S4096 (512 blocks, two a CU): whole by
+// length 1014, chunks 1156, whole head by head 1051 for the whole backward; S2048
+// (256 blocks): whole 358, chunks 308.
+KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, bool by_length, int cus) {
   const int64_t heads = (int64_t)batch * kv_heads;
   const int nkb = (nb + 1) / 2, longest = group * nb;
   auto per_head = [&](int chunk) {
@@ -653,7 +681,8 @@ KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, int cus)
   };
   KvPlan plan;
   plan.per_head = nkb;
-  double best = time(heads * nkb, longest);
+  double best = by_length ? 4 + 1.75 * std::max((double)longest, (double)total * heads / cus + 2)
+                          : time(heads * nkb, longest);
   for (int rounds = 1; rounds <= 3; ++rounds) {
     const int64_t most = (int64_t)rounds * cus / heads;
     if (most <= nkb)
@@ -697,10 +726,24 @@ hipError_t launch_bwd_dt(const BwdParams &p, bool sum, hipStream_t stream) {
                      stream, p);
   return hipGetLastError();
 }
+
+// Causal blocks go by length where the heads divide over the XCDs and what those
+// side by side read at once (rows of two tensors) is at most half the last-level
+// cache: with 256 MB (the dK/dV kernel's Q and dO of B8 H32 S2048) the backward
+// takes 1268 us head by head and 1375 by length, with 128 MB (B4) 649 and 610.
+// Smaller: B1 Hkv32 S1984 186 -> 145 us, B8 H16 S512 84 -> 71, B8 Hq32 Hkv8 S1024
+// 404 -> 321.
+bool by_length(int64_t heads, int64_t read_heads, int seq, bool causal) {
+  return causal && heads % 8 == 0 && read_heads * seq * (4 * kBD) <= (128 << 20);
+}
+bool kv_order(int batch, int q_heads, int kv_heads, int seq, bool causal) {
+  return by_length((int64_t)batch * kv_heads, (int64_t)batch * q_heads, seq, causal);
+}
 } // namespace
 
 size_t bwd_workspace_bytes(int batch, int q_heads, int kv_heads, int seq, bool causal, int cus) {
-  const KvPlan plan = kv_plan(batch, kv_heads, q_heads / kv_heads, seq / kBlk, causal, cus);
+  const KvPlan plan = kv_plan(batch, kv_heads, q_heads / kv_heads, seq / kBlk, causal,
+                              kv_order(batch, q_heads, kv_heads, seq, causal), cus);
   return plan.sum ? (size_t)batch * kv_heads * plan.per_head * kPartBytes : 0;
 }
 
@@ -724,8 +767,9 @@ hipError_t launch_bwd(const BwdArgs &a, hipStream_t stream) {
   p.scale = a.scale > 0.f ? a.scale : 1.0f / __builtin_sqrtf((float)kBD);
   p.scale_log2 = p.scale * kLog2eB;
   p.inv_scale = 1.0f / p.scale;
+  const bool kv_whole_order = kv_order(a.batch, a.q_heads, a.kv_heads, a.seq, a.causal != 0);
   KvPlan plan = kv_plan(a.batch, a.kv_heads, a.q_heads / a.kv_heads, a.seq / kBlk, a.causal != 0,
-                        a.cus);
+                        kv_whole_order, a.cus);
   if (plan.sum && (!a.workspace || a.workspace_bytes < (size_t)a.batch * a.kv_heads *
                                                            plan.per_head * kPartBytes)) {
     plan = KvPlan{};
@@ -734,6 +778,9 @@ hipError_t launch_bwd(const BwdArgs &a, hipStream_t stream) {
   p.chunk = plan.chunk;
   p.per_head = plan.per_head;
   p.part = static_cast<f32x4 *>(a.workspace);
+  p.kv_by_length = kv_whole_order && !plan.sum;
+  p.q_by_length = by_length((int64_t)a.batch * a.q_heads, (int64_t)a.batch * a.kv_heads, a.seq,
+                            a.causal != 0);
   if (a.dtype == kF16)
     return a.causal ? launch_bwd_dt<kF16, true>(p, plan.sum, stream)
                     : launch_bwd_dt<kF16, false>(p, plan.sum, stream);

@@ -168,3 +168,30 @@ def test_fa_bwd_work_split(wave, dev, dt, B, Hq, Hkv, S, causal):
         bound = ulp * y.double().abs() + 1e-5 * y.double().abs().max()
         assert bool((d <= bound).all()), f"{name}: {d.max().item()}"
         assert (d > 0).double().mean().item() < 0.05, f"{name}: {(d > 0).double().mean().item()}"
+
+
+# Causal blocks by length (heads a multiple of the 8 XCDs) against head by head
+# (each batch alone: 12 KV heads, 36 q heads): the same sums in the same order, so
+# the same bits.  One block, an odd number and an even number of 64-row blocks.
+@pytest.mark.parametrize("dt", [1, 2])
+@pytest.mark.parametrize("S", [64, 448, 1024])
+def test_fa_bwd_blocks_by_length(wave, dev, dt, S):
+    B, Hq, Hkv = 2, 36, 12
+    g = torch.Generator().manual_seed(41)
+    q, k, v, do = (torch.randn(s, generator=g).to(TDT[dt]).to(dev)
+                   for s in ((B, Hq, S, 128), (B, Hkv, S, 128), (B, Hkv, S, 128), (B, Hq, S, 128)))
+    o, lse = wave.flash_attention_lse(q, k, v, causal=True)
+
+    def grads(*t):  # one CTA a key block: without a workspace
+        out = [torch.full_like(x, float("nan")) for x in t[:3]]
+        wave.runtime.check(wave.runtime.lib().wave_fa_bwd_launch(
+            *(x.data_ptr() for x in (*t, torch.empty_like(t[5]), *out)), t[0].shape[0], Hq, Hkv, S,
+            128, dt, 1, 0.0, torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        return out
+
+    want = [torch.cat(x) for x in zip(*(grads(*(t[b:b + 1] for t in (q, k, v, o, do, lse)))
+                                        for b in range(B)))]
+    for name, x, y in zip(("dq", "dk", "dv"), grads(q, k, v, o, do, lse), want):
+        assert torch.equal(x, y), name
+    assert torch.equal(wave.flash_attention_bwd(q, k, v, o, do, lse, causal=True)[0], want[0])
