@@ -19,11 +19,10 @@
 // bytes each, 16-byte chunks XOR-swizzled by row so that the 32 rows of one
 // fragment read cover all banks); NS stages form a ring filled by
 // global->LDS DMA.  Wave w computes an RM x RN part of the block (WM x WN
-// waves) on 32x32x16 MFMAs, the fragments of slice kk + 1 read while slice kk
-// is multiplied.  One barrier a stage, before its last slice: there every
-// wave holds that slice in registers, so the barrier frees the stage's slot
-// for stage k + NS and publishes stage k + 1, whose first slice is read
-// under the last slice's MFMAs.
+// waves) on 32x32x16 MFMAs from one of two register sets: while stage k is
+// multiplied out of one, stage k + 1 is read into the other.  One barrier a
+// stage, at its start: there every wave holds stage k in registers, so the
+// barrier frees the slot for stage k + NS, and stage k + 1 has landed.
 //
 // Rows past M and N are fetched from the last valid row (their products only
 // reach elements of C that are never stored).  The K remainder (K % 64) is
@@ -65,7 +64,7 @@ struct BlockParams {
   float *slots;          // [tiles * splits][BM * BN] (splits > 1)
   u64 *counters;         // [tiles][2] arrived, published (epoch << 32 | count)
   uint32_t epoch;        // nonzero; the tag of this launch's counts
-  u64 *zero;             // zero_words words left zero (see GemmArgs)
+  u64 *zero;             // zero_words words left zero (BlockWorkspace)
   uint32_t zero_words;
 };
 
