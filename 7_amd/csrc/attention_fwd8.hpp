@@ -73,6 +73,7 @@ struct Fp8Params {
   int causal;
   float scale_log2;
   float *lse;
+  int by_length;  // causal CTA order (block_coords)
 };
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));
@@ -112,6 +113,7 @@ __device__ __forceinline__ void fwd8_cta(const Fp8Params &p, int raw, uint8_t *s
     cp.batch = p.batch;
     cp.q_heads = p.q_heads;
     cp.causal = CAUSAL;
+    cp.by_length = CAUSAL ? p.by_length : 0;
     block_coords(cp, raw, bh, qb);
   }
   const int b = bh / p.q_heads, hq = bh - b * p.q_heads;

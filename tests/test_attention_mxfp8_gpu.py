@@ -154,3 +154,23 @@ def test_rejections(wave, dev):
     kvs = torch.full((1, 3, 2, 128), 127, dtype=torch.uint8, device=dev)
     with pytest.raises(ValueError, match="multiple"):          # 2 q heads on 3 kv heads
         wave.flash_attention_mxfp8(q, s, kq, ks, kq, kvs)
+
+
+# Causal blocks by length (24 q heads, a multiple of the 8 XCDs) against head by
+# head (each batch alone: 12): every block is computed alike, so the same bits.
+@pytest.mark.parametrize("out_dt", [1, 2])
+@pytest.mark.parametrize("S", [1, 256, 1000, 3100])
+def test_blocks_by_length(wave, dev, out_dt, S):
+    g = torch.Generator(device=dev).manual_seed(S)
+    q, k, v = (torch.randn(2, h, S, 128, generator=g, device=dev) for h in (12, 4, 4))
+    t = [x for y in (wave.mxfp8_quantize(q), wave.mxfp8_quantize(k), wave.mxfp8_quantize(v, dim=2))
+         for x in y]
+
+    def attend(*t):
+        lse = torch.empty(t[0].shape[:3], device=dev)
+        return wave.flash_attention_mxfp8(*t, causal=True, out_dtype=ODT[out_dt], lse=lse), lse
+
+    o, lse = attend(*t)
+    parts = [attend(*(x[b:b + 1] for x in t)) for b in range(2)]
+    assert torch.equal(o, torch.cat([x[0] for x in parts]))
+    assert torch.equal(lse, torch.cat([x[1] for x in parts]))
