@@ -51,11 +51,13 @@ hipError_t launch_fwd(const FwdArgs &a, hipStream_t stream) {
                          (int64_t)a.batch * a.kv_heads * a.seq_k * (2 * kKRowBytes) <= (256 << 20);
   const bool narrow = a.waves == kPPWaves && (n128 <= (by_length ? 2 * a.cus : a.cus) ||
                                               (n256 > a.cus && 113 * n128 < 200 * n256));
-  p.by_length = !by_length ? 0 : !narrow ? 1 : n128 > a.cus ? std::max(a.cus / 8, 1) : 0;
   const int rows = a.waves == kR3Waves ? kR3Rows
                    : narrow            ? kF4PassRows
                                        : 32 * kPPWaves;  // 4 waves: two passes of 128
   p.q_blocks = (a.seq_q + rows - 1) / rows;
+  p.by_length = !by_length || p.q_blocks * heads <= a.cus ? 0
+                : narrow                                  ? std::max(a.cus / 8, 1)
+                                                          : 1;
   p.causal = a.causal;
   const float scale = a.scale > 0.f ? a.scale : 1.0f / std::sqrt((float)a.head_dim);
   p.scale_log2 = scale * kLog2e;
