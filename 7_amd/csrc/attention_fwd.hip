@@ -34,7 +34,7 @@ hipError_t launch_fwd(const FwdArgs &a, hipStream_t stream) {
   // ahead, B1 H61 S640 24.3 / 25.7).
   // Causal blocks are of uneven length: where the heads divide over the XCDs they
   // go by length (block_coords).  8-wave kernel, head by head -> by length:
-  // B4 Hq32 Hkv32 S3000 107 -> 84 us (B1), B4 H16 S2048 104 -> 78, B2 Hq32 Hkv8
+  // B1 Hq32 Hkv32 S3000 107 -> 84 us, B4 H16 S2048 104 -> 78, B2 Hq32 Hkv8
   // S4096 309 -> 277, B1 Hq64 Hkv8 S8192 1013 -> 979.  The heads then side by
   // side read their K and V at once, which the 256 MB last-level cache has to
   // hold: 32 MB in all (B1 Hq32 Hkv4 S16384) 1965 -> 1937 us, 256 MB (B4 H32
