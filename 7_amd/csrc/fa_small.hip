@@ -2,18 +2,26 @@
 // math of fa_small.hpp (the reference's single-workgroup kernel, which the
 // code objects keep) on a grid.
 //
-// A CTA owns 16 query rows x 16 TC output columns; its W waves deal the
-// 32-key blocks among themselves (wave w takes blocks w, w + W, ...), each with
-// its own running max, row sums and accumulators, and the results are merged
-// through LDS in wave order.  Nothing here is near a rate of the chip: the work
-// is a chain of load -> QK -> max -> exp2 -> PV steps, so its length is what
-// counts, and the loads of a wave's next block are in flight while it works on
-// the current one; V goes through LDS for the transposing read (gathered 2 bytes
-// a lane it took 13 us where this takes 9).  Measured (us, one workgroup / this
-// grid): 64 queries x 1024 keys x 64 130 / 9.0 (8 CTAs x 16 waves), 16 x 4096 x
-// 128 957 / 36, 4096 x 2048 x 128 11700 / 30.
+// A CTA owns 16 query rows x 16 TC output columns and takes the keys in rounds of
+// one 32-key block a wave.  Every result is, bit for bit, that of one wave going
+// through the blocks in order, which is what the single-workgroup kernel does:
+// the waves share the round's block maxima, so each rounds its probabilities
+// relative to the running max at its block, and the sums over blocks (rescale,
+// then one MFMA) are done in block order by one wave a column tile.  That chain
+// is short (about 45 cycles a block); scores, exp2 and loads are what the waves
+// do side by side.  (Waves with running maxima of their own, merged at the end,
+// round the probabilities otherwise: results 2e-4 away.)
+//
+// Nothing here is near a rate of the chip: a round is a chain of load -> QK ->
+// maxima -> exp2 -> PV steps, and the next round's loads are in flight during it.
+// Measured (us, one workgroup / this grid): 64 queries x 1024 keys x 64 130 / 8.5
+// (8 CTAs x 16 waves), 16 x 4096 x 128 957 / 36.5, 4096 x 2048 x 128 11700 / 30.
+// Keeping the query fragments in LDS lets the D = 128 step fit 128 registers
+// (with them in registers it spilled: 16 x 4096 x 128 47.8; 64 x 1024 x 64 10.9).
 #include "attention.hpp"
 #include "fa_small.hpp"
+
+#include <type_traits>
 
 namespace wave {
 namespace attention {
@@ -30,211 +38,266 @@ template <int TC> constexpr int max_waves() { return TC > 2 ? kSplitWaves / 2 : 
 template <int ND, int TC>
 __global__ __launch_bounds__(64 * max_waves<TC>()) void small_split_kernel(
     const _Float16 *Q, const _Float16 *K, const _Float16 *V, float *O, int block_m, int seq_n,
-    int D, int col_units) {
+    int D, int col_units, uint32_t units) {
   constexpr int NF = ND > 0 ? ND : 1;
   constexpr int MAXW = max_waves<TC>();
-  // A wave's LDS: its V block of 32 keys x 16 TC columns (ND > 0), then, after
-  // the loop, its sums -- both 1 KiB a tile, and no other wave's.
-  __shared__ f32x4 part[MAXW][TC][64];
-  __shared__ float wave_m[MAXW][16], wave_l[MAXW][16];
+  // What the waves leave for a round's chain, by key block: V (32 keys x 16 TC
+  // columns; ND = 0: TC operands of 64 lanes), P as the product's operand, each
+  // lane's sum of its P, each query's factor of the earlier sums and block max.
+  __shared__ f32x4 sv[MAXW][TC][64];
+  __shared__ u32x4 sp[MAXW][64], sq[NF][64];
+  __shared__ float ssum[MAXW][64], salpha[MAXW][16];
+  __shared__ __attribute__((aligned(16))) float smax[16][MAXW + 4];  // padded: no bank conflicts
+  const uint32_t unit = blockIdx.y * gridDim.x + blockIdx.x;
+  if (unit >= units)
+    return;  // the whole CTA
   const int W = blockDim.x >> 6, wave = (int)uniform(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
-  const int unit = blockIdx.x;
-  const int q0 = unit / col_units * 16, c0 = unit % col_units * (16 * TC);
+  const int q0 = (int)(unit / col_units) * 16, c0 = (int)(unit % col_units) * (16 * TC);
   const int qrow = q0 + col;
   const bool q_ok = qrow < block_m;
   const uint16_t *vh = reinterpret_cast<const uint16_t *>(V);
   const u32x4 zero4 = {0u, 0u, 0u, 0u};
 
-  // 8 halves of row `row` (valid) at column d, zero past D.
-  auto chunk = [&](const _Float16 *base, int row, int d) {
-    return d < D ? *reinterpret_cast<const u32x4 *>(base + (size_t)row * D + d) : zero4;
+  // 8 halves of row min(row, rows) at column d (d a multiple of 8), zero past the
+  // rows and past D: those lanes read past the buffer, which gives zeros ((rows +
+  // 1) * D < 2^30, so the bytes of row `rows` lie below 2^31).
+  auto rsrc = [&](const _Float16 *base, int rows) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16 *>(base), 0,
+                                             (uint32_t)rows * (uint32_t)D * 2u, 0x00020000);
   };
-  u32x4 qf[NF];
-  if constexpr (ND > 0) {
-#pragma unroll
-    for (int s = 0; s < ND; ++s)
-      qf[s] = q_ok ? chunk(Q, qrow, 32 * s + 8 * grp) : zero4;
-  }
+  const uint32_t pitch = (uint32_t)D * 2u;
+  auto past = [&](int d) { return (uint32_t)((D - 8 - d) >> 31) & 0x80000000u; };
+  auto chunk = [&](__amdgpu_buffer_rsrc_t r, int rows, int row, int d) {
+    const uint32_t at = (uint32_t)min(row, rows) * pitch + ((uint32_t)d * 2u + past(d));
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0));
+  };
+  const __amdgpu_buffer_rsrc_t rk = rsrc(K, seq_n), rv = rsrc(V, seq_n);
 
   // One block's operands: K rows n0 + 16h + col and, as rows of 16-byte pieces
   // (ND > 0), V; piece i of a lane is row (lane + 64 i) / (2 TC), chunk
   // (lane + 64 i) % (2 TC).
-  struct Block {
-    u32x4 k[2][NF], v[TC];
-  };
-  auto load = [&](Block &b, int n0) {
+  u32x4 kf[2][NF], vf[TC];
+  auto load_k = [&](int n0) {
     if constexpr (ND > 0) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int key = min(n0 + 16 * h + col, seq_n - 1);  // masked below
+        const int key = n0 + 16 * h + col;
 #pragma unroll
         for (int s = 0; s < ND; ++s)
-          b.k[h][s] = chunk(K, key, 32 * s + 8 * grp);
+          kf[h][s] = chunk(rk, seq_n, key, 32 * s + 8 * grp);
       }
+    }
+  };
+  auto load_v = [&](int n0) {
+    if constexpr (ND > 0) {
 #pragma unroll
       for (int i = 0; i < TC; ++i) {
         const int piece = lane + 64 * i, key = n0 + piece / (2 * TC);
-        b.v[i] = key < seq_n ? chunk(V, key, c0 + 8 * (piece % (2 * TC))) : zero4;
+        vf[i] = chunk(rv, seq_n, key, c0 + 8 * (piece % (2 * TC)));
       }
     }
   };
-  // V^T as the PV product's A operand: column c0 + 16t + col, keys in the order
-  // the scores come out (4 grp + 0..3, 16 + 4 grp + 0..3).  ND > 0: through the
-  // transposing LDS read (lane 16g + i of a group receives element i of the
-  // four rows that lanes 16g + 4j + 0..3 address), else gathered.
   auto key_of = [&](int n0, int j) { return n0 + (j < 4 ? 4 * grp + j : 16 + 4 * grp + j - 4); };
+  auto store_v = [&](int n0) {
+#pragma unroll
+    for (int i = 0; i < TC; ++i) {
+      if constexpr (ND > 0) {
+        sv[wave][i][lane] = __builtin_bit_cast(f32x4, vf[i]);
+      } else {
+        const int c = c0 + 16 * i + col;
+        u32x4 w = zero4;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int key = key_of(n0, j);
+          const uint32_t x = vh[(size_t)min(key, seq_n - 1) * D + min(c, D - 1)];
+          w[j >> 1] |= (key < seq_n && c < D ? x : 0u) << (16 * (j & 1));
+        }
+        sv[wave][i][lane] = __builtin_bit_cast(f32x4, w);
+      }
+    }
+  };
+  // V^T of block b of the round as the PV product's A operand: column c0 + 16t +
+  // col, keys in the order the scores come out (4 grp + 0..3, 16 + 4 grp + 0..3).
+  // ND > 0: through the transposing LDS read (lane 16g + i of a group receives
+  // element i of the four rows that lanes 16g + 4j + 0..3 address).
   typedef short s16x4 __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const uint32_t vbase = lds_addr(part) + wave * (TC * 1024);
-  auto store_v = [&](const Block &b) {
-#pragma unroll
-    for (int i = 0; i < TC; ++i)
-      part[wave][i][lane] = __builtin_bit_cast(f32x4, b.v[i]);
-  };
-  auto v_operand = [&](int t, int n0) {
+  const uint32_t vbase = lds_addr(sv) + (4 * grp + (col >> 2)) * (32 * TC) + 8 * (col & 3);
+  auto v_operand = [&](int b, int t) {
     if constexpr (ND > 0) {
-      const uint32_t row = 4 * grp + (col >> 2);
-      const uint32_t at = vbase + row * (32 * TC) + 32 * t + 8 * (col & 3);
+      const uint32_t at = vbase + b * (TC * 1024) + 32 * t;
       const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(uintptr_t)at);
       const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
           (lds_s16x4 *)(uintptr_t)(at + 16 * 32 * TC));
-      const u32x2 a = __builtin_bit_cast(u32x2, lo), b = __builtin_bit_cast(u32x2, hi);
-      return u32x4{a[0], a[1], b[0], b[1]};
+      const u32x2 x = __builtin_bit_cast(u32x2, lo), y = __builtin_bit_cast(u32x2, hi);
+      return u32x4{x[0], x[1], y[0], y[1]};
     } else {
-      const int c = c0 + 16 * t + col;
-      u32x4 w = zero4;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int key = key_of(n0, j);
-        const uint32_t x = vh[(size_t)min(key, seq_n - 1) * D + min(c, D - 1)];
-        w[j >> 1] |= (key < seq_n && c < D ? x : 0u) << (16 * (j & 1));
-      }
-      return w;
+      return __builtin_bit_cast(u32x4, sv[b][t][lane]);
     }
   };
 
-  f32x4 acc[TC];
-#pragma unroll
-  for (int t = 0; t < TC; ++t)
-    acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Waves 0 .. TC-1 carry a column tile each (W >= TC) through the chain.
+  const bool carries = wave < TC && c0 + 16 * wave < D;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   float m = -__builtin_inff(), l = 0.f;
-  const int step = 32 * W;
-  Block cur, nxt;
-  load(cur, 32 * wave);  // W <= blocks: every wave has one
-  for (int n0 = 32 * wave; n0 < seq_n; n0 += step) {
-    if (n0 + step < seq_n)
-      load(nxt, n0 + step);
-    if constexpr (ND > 0) {
-      // The previous block's reads of this LDS are done (its values are in
-      // MFMA operands); the stores below land before this block's reads.
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      store_v(cur);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  const int blocks = (seq_n - 1) / 32 + 1;
+  // The query fragments, the same for every wave: in LDS, not 4 ND registers.
+  u32x4 qr[NF];
+  if constexpr (ND > 0) {
+    if (wave == 0) {
+#pragma unroll
+      for (int s = 0; s < ND; ++s)
+        qr[s] = chunk(rsrc(Q, block_m), block_m, qrow, 32 * s + 8 * grp);
     }
-    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-    auto qk = [&](int h, u32x4 kf, u32x4 q) {
-      s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, kf),
-                                                    __builtin_bit_cast(f16x8, q), s[h], 0, 0, 0);
-    };
-    if constexpr (ND > 0) {
+  }
+  load_k(32 * wave);
+  load_v(32 * wave);
+  if constexpr (ND > 0) {
+    if (wave == 0) {
 #pragma unroll
-      for (int d = 0; d < ND; ++d)
+      for (int s = 0; s < ND; ++s)
+        sq[s][lane] = qr[s];
+    }
+    lds_barrier();
+  }
+  for (int b0 = 0; b0 < blocks; b0 += W) {
+    const int here = min(W, blocks - b0);  // the round's blocks
+    const bool mine = wave < here;
+    const int n0 = (int)(32u * (uint32_t)(b0 + wave));
+    float p[8], top = -__builtin_inff();
+    if (mine) {
+      f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+      auto qk = [&](int h, u32x4 k, u32x4 q) {
+        s[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, k),
+                                                      __builtin_bit_cast(f16x8, q), s[h], 0, 0, 0);
+      };
+      if constexpr (ND > 0) {
+        u32x4 q[NF];
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-          qk(h, cur.k[h][d], qf[d]);
-    } else {
-      for (int d0 = 0; d0 < D; d0 += 32) {
-        const u32x4 q = small_load8(Q, qrow, q_ok, d0 + 8 * grp, D, D);
+        for (int d = 0; d < ND; ++d)
+          q[d] = sq[d][lane];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int key = n0 + 16 * h + col;
-          qk(h, small_load8(K, key, key < seq_n, d0 + 8 * grp, D, D), q);
+        for (int d = 0; d < ND; ++d)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            qk(h, kf[h][d], q[d]);
+      } else {
+        for (int d0 = 0; d0 < D; d0 += 32) {
+          const u32x4 q = small_load8(Q, qrow, q_ok, d0 + 8 * grp, D, D);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int key = n0 + 16 * h + col;
+            qk(h, small_load8(K, key, key < seq_n, d0 + 8 * grp, D, D), q);
+          }
         }
       }
-    }
-    float p[8], cmax = -__builtin_inff();
+      load_k(n0 + 32 * W);  // the next round's, early; zeros past the last key
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      p[j] = key_of(n0, j) < seq_n ? s[j >> 2][j & 3] : -__builtin_inff();
-      cmax = fmaxf(cmax, p[j]);
+      for (int j = 0; j < 8; ++j) {
+        p[j] = key_of(n0, j) < seq_n ? s[j >> 2][j & 3] : -__builtin_inff();
+        top = fmaxf(top, p[j]);
+      }
+      top = small_wave_max4(top);
+      if (grp == 0)
+        smax[col][wave] = top;
     }
-    const float m_new = fmaxf(m, small_wave_max4(cmax));
-    // A wave whose scores are all -inf so far contributes nothing (another
-    // wave's may be finite).
-    const float base = m_new == -__builtin_inff() ? 0.f : m_new;
-    const float alpha = exp2f(m - base);
-    m = m_new;
-    float psum = 0.f;
+    lds_barrier();  // the round's maxima; the last round's chain is done
+    float before = m;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      p[j] = exp2f(p[j] - base);
-      psum += p[j];
-    }
-    l = l * alpha + psum;
-    const u32x4 pf = {small_pack_f16(p[0], p[1]), small_pack_f16(p[2], p[3]),
-                      small_pack_f16(p[4], p[5]), small_pack_f16(p[6], p[7])};
+    for (int w4 = 0; w4 < MAXW; w4 += 4) {
+      const f32x4 x = *reinterpret_cast<const f32x4 *>(&smax[col][w4]);
 #pragma unroll
-    for (int t = 0; t < TC; ++t) {
-      acc[t] *= alpha;
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-          __builtin_bit_cast(f16x8, v_operand(t, n0)), __builtin_bit_cast(f16x8, pf), acc[t], 0, 0,
-          0);
+      for (int i = 0; i < 4; ++i) {
+        before = fmaxf(before, w4 + i < wave ? x[i] : -__builtin_inff());
+        m = fmaxf(m, w4 + i < here ? x[i] : -__builtin_inff());
+      }
     }
-    cur = nxt;
+    if (mine) {
+      const float m_new = fmaxf(before, top);
+      float psum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        p[j] = exp2f(p[j] - m_new);
+        psum += p[j];
+      }
+      sp[wave][lane] = u32x4{small_pack_f16(p[0], p[1]), small_pack_f16(p[2], p[3]),
+                             small_pack_f16(p[4], p[5]), small_pack_f16(p[6], p[7])};
+      ssum[wave][lane] = psum;
+      if (grp == 0)
+        salpha[wave][col] = exp2f(before - m_new);
+      store_v(n0);
+      load_v(n0 + 32 * W);
+    }
+    lds_barrier();  // the round's P, V, sums and factors
+    if (carries) {
+      // N blocks from b on: their operands read together, then multiplied in order.
+      auto chain = [&](int b, auto group) {
+        constexpr int N = decltype(group)::value;
+        u32x4 pb[N], vb[N];
+        float alpha[N], psum[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          alpha[i] = salpha[b + i][col];
+          psum[i] = ssum[b + i][lane];
+          pb[i] = sp[b + i][lane];
+          vb[i] = v_operand(b + i, wave);
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          l = l * alpha[i] + psum[i];
+          acc *= alpha[i];
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, vb[i]),
+                                                       __builtin_bit_cast(f16x8, pb[i]), acc, 0, 0,
+                                                       0);
+        }
+      };
+      constexpr int G = ND == 4 && TC == 2 ? 2 : 4;  // what the registers hold
+      int b = 0;
+#pragma unroll 1
+      for (; b + G <= here; b += G)
+        chain(b, std::integral_constant<int, G>{});
+#pragma unroll 1
+      for (; b < here; ++b)
+        chain(b, std::integral_constant<int, 1>{});
+    }
   }
-
-  // Merge: O = sum_w 2^(m_w - m) acc_w / sum_w 2^(m_w - m) l_w, in wave order.
-  l = small_wave_sum4(l);
-  if (grp == 0) {
-    wave_m[wave][col] = m;
-    wave_l[wave][col] = l;
-  }
+  if (!carries)
+    return;
+  const float inv = 1.0f / small_wave_sum4(l);
+  if (!q_ok)
+    return;
+  // O^T rows are output columns: registers hold columns 4 grp .. +3.
+  const int c = c0 + 16 * wave + 4 * grp;
 #pragma unroll
-  for (int t = 0; t < TC; ++t)
-    part[wave][t][lane] = acc[t];
-  __syncthreads();
-  float top = -__builtin_inff();
-  for (int w = 0; w < W; ++w)
-    top = fmaxf(top, wave_m[w][col]);
-  float total = 0.f;
-  for (int w = 0; w < W; ++w)
-    total += wave_l[w][col] * exp2f(wave_m[w][col] - top);
-  const float inv = 1.0f / total;
-  for (int t = wave; t < TC; t += W) {
-    f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    for (int w = 0; w < W; ++w)
-      o += part[w][t][lane] * exp2f(wave_m[w][col] - top);
-    // O^T rows are output columns: registers hold columns 4 grp .. +3.
-    const int c = c0 + 16 * t + 4 * grp;
-    if (q_ok) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (c + i < D)
-          O[(size_t)qrow * D + c + i] = o[i] * inv;
-    }
-  }
+  for (int i = 0; i < 4; ++i)
+    if (c + i < D)
+      O[(size_t)qrow * D + c + i] = acc[i] * inv;
 }
 
 template <int TC>
 hipError_t launch_tc(const _Float16 *Q, const _Float16 *K, const _Float16 *V, float *O, int block_m,
                      int seq_n, int D, hipStream_t stream) {
   const int blocks = (seq_n - 1) / 32 + 1, most = max_waves<TC>();
-  const int waves = blocks < most ? blocks : most;
+  const int waves = blocks < TC ? TC : blocks < most ? blocks : most;
   const int col_units = (D - 1) / (16 * TC) + 1;
-  const dim3 grid((unsigned)((block_m - 1) / 16 + 1) * (unsigned)col_units), block(64 * waves);
-  const bool vec = D % 8 == 0 && ((reinterpret_cast<uintptr_t>(Q) |
-                                   reinterpret_cast<uintptr_t>(K) |
-                                   reinterpret_cast<uintptr_t>(V)) & 15) == 0;
+  // At most 2^27 units (block_m * D < 2^31); a grid dimension holds fewer than 2^32
+  // threads.
+  const uint32_t units = ((uint32_t)(block_m - 1) / 16 + 1) * (uint32_t)col_units, row = 1u << 21;
+  const dim3 grid(units < row ? units : row, (units - 1) / row + 1), block(64 * waves);
+  const int64_t rows = (int64_t)(block_m > seq_n ? block_m : seq_n) + 1;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) |
+                       reinterpret_cast<uintptr_t>(V);
+  const bool vec = D % 8 == 0 && at % 16 == 0 && rows * D < (1 << 30);
   if (vec && D <= 64)
     hipLaunchKernelGGL((small_split_kernel<2, TC>), grid, block, 0, stream, Q, K, V, O, block_m,
-                       seq_n, D, col_units);
+                       seq_n, D, col_units, units);
   else if (vec && D <= 128)
     hipLaunchKernelGGL((small_split_kernel<4, TC>), grid, block, 0, stream, Q, K, V, O, block_m,
-                       seq_n, D, col_units);
+                       seq_n, D, col_units, units);
   else
     hipLaunchKernelGGL((small_split_kernel<0, TC>), grid, block, 0, stream, Q, K, V, O, block_m,
-                       seq_n, D, col_units);
+                       seq_n, D, col_units, units);
   return hipGetLastError();
 }
 
