@@ -291,7 +291,7 @@ def _eager_device_tensor(x: torch.Tensor) -> bool:
     """Whether x is a plain device tensor outside any tracing or transform, so
     that its pointer is what the operation runs on."""
     return (x.is_cuda and type(x) in (torch.Tensor, torch.nn.Parameter)
-            and not torch.compiler.is_compiling()
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
             and not torch._C._functorch.is_functorch_wrapped_tensor(x)
             and torch._C._len_torch_dispatch_stack() == 0)
 

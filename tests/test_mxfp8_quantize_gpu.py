@@ -105,3 +105,11 @@ def test_other_dtypes_and_graphs(wave, dev):
         torch.cuda.synchronize()
         we, ws = wave.mxfp8_quantize(h)
         assert torch.equal(e, we) and torch.equal(sc, ws)
+
+
+def test_jit_trace_is_refused(wave, dev):
+    """A trace would record the output allocations without the launch between
+    them; it takes the formula, whose uint8 views torch.jit.trace refuses."""
+    x = values((4, 64), torch.float32, 9).to(dev)
+    with pytest.raises(RuntimeError):
+        torch.jit.trace(lambda t: wave.mxfp8_quantize(t), (x,), check_trace=False)
