@@ -113,3 +113,22 @@ def test_jit_trace_is_refused(wave, dev):
     x = values((4, 64), torch.float32, 9).to(dev)
     with pytest.raises(RuntimeError):
         torch.jit.trace(lambda t: wave.mxfp8_quantize(t), (x,), check_trace=False)
+
+
+@pytest.mark.parametrize("dim", [0, 1])
+def test_lazy_tensors(wave, dev, dim):
+    """Views that are negated when read, and zero tensors without memory."""
+    x = values((64, 96), torch.float32, 10).nan_to_num().to(dev)
+    neg = torch._neg_view(x)
+    assert neg.is_neg()
+    for got, want in zip(wave.mxfp8_quantize(neg, dim), wave.mxfp8_quantize(-x, dim)):
+        assert torch.equal(got, want)
+    # The imaginary part of a conjugate: negated and strided.
+    z = torch.complex(x, x.flip(0)).conj().imag
+    assert z.is_neg()
+    for got, want in zip(wave.mxfp8_quantize(z, dim), wave.mxfp8_quantize(-x.flip(0), dim)):
+        assert torch.equal(got, want)
+    zero = torch._efficientzerotensor((64, 96), device=dev)
+    for got, want in zip(wave.mxfp8_quantize(zero, dim),
+                         wave.mxfp8_quantize(torch.zeros((64, 96), device=dev), dim)):
+        assert torch.equal(got, want)
