@@ -111,10 +111,20 @@ __device__ __forceinline__ void encode(const float (&v)[N], uint32_t amax, float
     out[i] = pack4(v[4 * i] * inv, v[4 * i + 1] * inv, v[4 * i + 2] * inv, v[4 * i + 3] * inv);
 }
 
+// Blocks in two grid dimensions: one holds fewer than 2^32 threads.
+dim3 grid_of(size_t blocks) {
+  constexpr size_t kRow = (size_t)1 << 22;
+  return blocks <= kRow ? dim3((unsigned)blocks)
+                        : dim3((unsigned)kRow, (unsigned)((blocks + kRow - 1) / kRow));
+}
+__device__ __forceinline__ size_t linear_block() {
+  return (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+}
+
 template <int DT>
 __global__ __launch_bounds__(256) void rows_kernel(const uint8_t *X, uint8_t *E, uint8_t *S,
                                                    size_t halves) {
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t t = linear_block() * 256 + threadIdx.x;
   if (t >= halves)
     return;  // halves is even: lane pairs stay whole
   constexpr int NW = 16 * elem_bytes<DT>() / 4;
@@ -149,14 +159,14 @@ __global__ __launch_bounds__(256) void cols_kernel(const uint8_t *X, uint8_t *E,
                                                    uint32_t units, uint32_t n, uint32_t blocks,
                                                    uint32_t groups) {
   const uint32_t lane = threadIdx.x & 63;
-  const uint32_t u = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 32 + (lane & 31);
+  const size_t u = (linear_block() * 4 + (threadIdx.x >> 6)) * 32 + (lane & 31);
   if (u >= units)
     return;  // both halves of a unit leave together
-  const uint32_t ob = u / groups, cg = u - ob * groups;
+  const uint32_t ob = (uint32_t)u / groups, cg = (uint32_t)u - ob * groups;
   const uint32_t o = ob / blocks, blk = ob - o * blocks;
   const uint32_t row0 = blk * kBlock + (lane >> 5) * 16;
-  const size_t inner = (size_t)groups * 4;
-  const size_t base = ((size_t)o * n + row0) * inner + cg * 4;
+  const size_t inner = (size_t)groups * 4, col = (size_t)cg * 4;
+  const size_t base = ((size_t)o * n + row0) * inner + col;
   const uint32_t rows = row0 < n ? min(n - row0, 16u) : 0u;
   constexpr int NW = elem_bytes<DT>();  // dwords of 4 values
   uint32_t w[16][NW];
@@ -216,14 +226,14 @@ __global__ __launch_bounds__(256) void cols_kernel(const uint8_t *X, uint8_t *E,
     }
   }
   if (lane < 32)
-    *reinterpret_cast<uint32_t *>(S + (size_t)ob * inner + cg * 4) = scales;
+    *reinterpret_cast<uint32_t *>(S + (size_t)ob * inner + col) = scales;
 }
 
 template <int DT>
 __global__ __launch_bounds__(256) void any_kernel(const void *X, uint8_t *E, uint8_t *S,
                                                   size_t total, size_t n, size_t blocks,
                                                   size_t inner) {
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;  // (outer, block, inner)
+  const size_t t = linear_block() * 256 + threadIdx.x;  // (outer, block, inner)
   if (t >= total)
     return;
   const size_t ob = t / inner, i = t - ob * inner;
@@ -255,18 +265,18 @@ hipError_t launch_dt(const void *X, void *E, void *S, size_t outer, size_t n, si
   if (inner == 1 && n % kBlock == 0 && (xa | ea) % 16 == 0 &&
       outer * n / 16 < ((size_t)1 << 39)) {
     threads = outer * n / 16;
-    hipLaunchKernelGGL((rows_kernel<DT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+    hipLaunchKernelGGL((rows_kernel<DT>), grid_of((threads + 255) / 256), dim3(256), 0,
                        stream, x, e, s, threads);
   } else if (inner % 4 == 0 && n < ((size_t)1 << 31) && units < ((size_t)1 << 31) &&
              xa % (4 * elem_bytes<DT>()) == 0 && (ea | sa) % 4 == 0) {
-    hipLaunchKernelGGL((cols_kernel<DT>), dim3((unsigned)((units + 127) / 128)), dim3(256), 0,
+    hipLaunchKernelGGL((cols_kernel<DT>), grid_of((units + 127) / 128), dim3(256), 0,
                        stream, x, e, s, (uint32_t)units, (uint32_t)n, (uint32_t)blocks,
                        (uint32_t)groups);
   } else {
     threads = outer * blocks * inner;
     if (threads >= ((size_t)1 << 39))
       return hipErrorInvalidValue;
-    hipLaunchKernelGGL((any_kernel<DT>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+    hipLaunchKernelGGL((any_kernel<DT>), grid_of((threads + 255) / 256), dim3(256), 0,
                        stream, X, e, s, threads, n, blocks, inner);
   }
   return hipGetLastError();

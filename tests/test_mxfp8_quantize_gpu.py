@@ -132,3 +132,23 @@ def test_lazy_tensors(wave, dev, dim):
     for got, want in zip(wave.mxfp8_quantize(zero, dim),
                          wave.mxfp8_quantize(torch.zeros((64, 96), device=dev), dim)):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dim", [0, 1])
+def test_beyond_32_bits(wave, dev, dim):
+    """2^32 + 64 blocks of one value: columns past 2^32 (across), and more blocks
+    than one grid dimension holds threads for (along)."""
+    n, part = (1 << 32) + 64, 1 << 20
+    x = torch.full((n,), 1.5, dtype=torch.bfloat16, device=dev)
+    ends = (slice(0, part), slice((1 << 31) - part, 1 << 31), slice(n - part, n))
+    for i, at in enumerate(ends):
+        x[at] = values((part,), torch.bfloat16, 11 + i).nan_to_num().to(dev)
+    got = [t.view(n) for t in wave.mxfp8_quantize(x.view((1, n) if dim == 0 else (n, 1)), dim)]
+    for at in ends:
+        want = wave.ops._mxfp8_quantize_formula(x[at].view((1, part) if dim == 0 else (part, 1)),
+                                                dim)
+        for a, b in zip(got, want):
+            assert torch.equal(a[at], b.view(part))
+    # 1.5 = 384 * 2^-8, everywhere between.
+    assert bool((got[0][part:(1 << 31) - part] == 0x7C).all())
+    assert bool((got[1][1 << 31:n - part] == 127 - 8).all())
