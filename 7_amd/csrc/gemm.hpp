@@ -60,14 +60,21 @@ GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, int workers,
                    const SplitLimits &limits);
 bool rows_vec4(const GemmArgs &args);
 // A small-block launch: `slots` / `counters` for splits > 1 (any contents: a
-// counter word counts only under this launch's nonzero `epoch`; left zero),
+// counter word counts only under this launch's `tag`; left zero),
 // and zero_words 64-bit words at `zero` left zero.
 struct BlockWorkspace {
   float *slots = nullptr;
   unsigned long long *counters = nullptr, *zero = nullptr;
   size_t zero_words = 0;
-  uint32_t epoch = 0;
+  uint64_t tag = 0;  // split_tag()
 };
+// Counts share a word with their launch's tag: the low bits, up to kMaxSplits.
+constexpr unsigned long long kCountMask = 15;
+constexpr int kMaxSplits = 8;
+static_assert(kMaxSplits <= (int)kCountMask, "a count fits its bits");
+// A tag for one split launch: nonzero, kCountMask's bits zero, the others drawn
+// anew each time (any thread).
+uint64_t split_tag();
 hipError_t launch_blocks(const GemmArgs &args, const GemmPlan &plan, const BlockWorkspace &ws,
                          hipStream_t stream);
 

@@ -37,10 +37,12 @@
 // themselves published; the last waits for that count, reads the partials
 // with device-coherent loads and sums them in split order (its own from its
 // accumulators), so the result does not depend on arrival order.  Counter
-// words are 64-bit: the launch's epoch (nonzero, from the host) in the high
-// half, a count in the low half; a word with any other epoch counts as zero,
-// so a workspace needs no clearing, and the last arriver leaves zeros, which
-// keeps replays of a captured launch (a fixed epoch) correct.
+// words are 64-bit: the launch's tag (split_tag(), nonzero) in the high 60 bits,
+// a count in the low four; a word with any other tag counts as zero, so a
+// workspace needs no clearing, and the last arriver leaves zeros, which keeps
+// replays of a captured launch (a fixed tag) correct.  Tags are drawn from all
+// of their 60 bits, so a word that holds anything else (partial sums of another
+// shape, recycled memory) matches with a chance of 2^-60.
 
 #include "gemm.hpp"
 #include "gemm_kernels.hpp"
@@ -62,8 +64,8 @@ struct BlockParams {
   int tiles_m, tiles_n, group_m;
   int splits;
   float *slots;          // [tiles * splits][BM * BN] (splits > 1)
-  u64 *counters;         // [tiles][2] arrived, published (epoch << 32 | count)
-  uint32_t epoch;        // nonzero; the tag of this launch's counts
+  u64 *counters;         // [tiles][2] arrived, published (tag | count)
+  u64 tag;               // split_tag() of this launch
   u64 *zero;             // zero_words words left zero (BlockWorkspace)
   uint32_t zero_words;
 };
@@ -95,18 +97,18 @@ template <int BM_, int BN_> struct BlockCfg {
 
 __device__ __forceinline__ uint32_t sw8(uint32_t r) { return (r ^ (r >> 3)) & 7u; }
 
-__device__ __forceinline__ uint32_t epoch_count(u64 w, uint32_t epoch) {
-  return (uint32_t)(w >> 32) == epoch ? (uint32_t)w : 0u;
+__device__ __forceinline__ uint32_t tag_count(u64 w, u64 tag) {
+  return (w & ~kCountMask) == tag ? (uint32_t)(w & kCountMask) : 0u;
 }
 // Counts one arrival on *c for this launch and returns the count before it.
 // The first guess is the zero every launch leaves, so the common first
 // arrival takes one atomic round trip; each failed exchange means another
 // contributor's succeeded (at most splits - 1) or the word was stale.
-__device__ __forceinline__ uint32_t epoch_increment(u64 *c, uint32_t epoch) {
+__device__ __forceinline__ uint32_t tag_increment(u64 *c, u64 tag) {
   u64 old = 0;
   for (;;) {
-    const uint32_t n = epoch_count(old, epoch);
-    if (__hip_atomic_compare_exchange_strong(c, &old, ((u64)epoch << 32) | (n + 1u),
+    const uint32_t n = tag_count(old, tag);
+    if (__hip_atomic_compare_exchange_strong(c, &old, tag | (n + 1u),
                                              __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT))
       return n;
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(256, X::OCC) void block_kernel(BlockParams p) {
     uint32_t *arrival = reinterpret_cast<uint32_t *>(smem);
     __syncthreads();
     if (threadIdx.x == 0)
-      *arrival = epoch_increment(&p.counters[2 * tile], p.epoch);
+      *arrival = tag_increment(&p.counters[2 * tile], p.tag);
     __syncthreads();
     if (*arrival != (uint32_t)p.splits - 1) {
       const __amdgpu_buffer_rsrc_t mine =
@@ -384,19 +386,19 @@ __global__ __launch_bounds__(256, X::OCC) void block_kernel(BlockParams p) {
       // the barrier, so thread 0's count, issued after it, needs no release.
       vm_wait_barrier();
       if (threadIdx.x == 0)
-        epoch_increment(&p.counters[2 * tile + 1], p.epoch);
+        tag_increment(&p.counters[2 * tile + 1], p.tag);
       return;
     }
     // Every other contributor has its ticket, so it is resident and publishes
     // without waiting on anything: the wait ends.  It is bounded all the same
     // (2^20 polls, about a second), for a counter word that already held this
-    // launch's epoch (a chance of 2^-32 a word for arbitrary contents).
+    // launch's tag (a chance of 2^-60 a word for arbitrary contents).
     if (threadIdx.x == 0) {
       for (uint32_t poll = 0;
            poll < (1u << 20) &&
-           epoch_count(__hip_atomic_load(&p.counters[2 * tile + 1], __ATOMIC_RELAXED,
+           tag_count(__hip_atomic_load(&p.counters[2 * tile + 1], __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT),
-                       p.epoch) != (uint32_t)p.splits - 1;
+                     p.tag) != (uint32_t)p.splits - 1;
            ++poll)
         __builtin_amdgcn_s_sleep(1);
       __hip_atomic_store(&p.counters[2 * tile], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -7,7 +7,11 @@
 #define WAVE_GEMM_GROUP_M 4
 #endif
 
+#include <sys/random.h>
+
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <type_traits>
 #include <vector>
 
@@ -139,7 +143,6 @@ constexpr BlockCost kBlocks[] = {
 // others (1000^2 x 1001 60.3 us in tiles, 15.8 in blocks; 2048^2 59.8 / 32.7;
 // 3000^2 62.8 / about 70).
 constexpr float kMaskedTile = 3.4f, kMaskedBlock = .8f, kMaskedShared = .46f;
-constexpr int kMaxSplits = 8;
 constexpr int kMinSplitStages = 4;  // stages a split keeps
 
 int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -255,10 +258,32 @@ size_t short_m_counter_count(int N, const SplitPlan &plan) {
   return 2 * (size_t)((N + plan.bn - 1) / plan.bn);
 }
 
+uint64_t split_tag() {
+  // A counter through the output function of SplitMix64 (Steele, Lea, Flood 2014),
+  // a bijection that spreads it over all 64 bits; its start comes from the
+  // kernel's random source, or the clock and an address.
+  static std::atomic<uint64_t> state{[] {
+    uint64_t seed = 0;
+    if (getrandom(&seed, sizeof seed, GRND_NONBLOCK) != (ssize_t)sizeof seed)
+      seed = (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() ^
+             (uint64_t)(uintptr_t)&seed << 20;
+    return seed;
+  }()};
+  for (;;) {
+    uint64_t z = state.fetch_add(0x9E3779B97F4A7C15ull, std::memory_order_relaxed);
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    z = (z ^ (z >> 31)) & ~(uint64_t)kCountMask;
+    if (z)
+      return z;
+  }
+}
+
 hipError_t launch_blocks(const GemmArgs &g, const GemmPlan &plan, const BlockWorkspace &ws,
                          hipStream_t stream) {
   if (plan.bm == 0 || plan.splits < 1 ||
-      (plan.splits > 1 && (!ws.slots || !ws.counters || !ws.epoch || g.K / 64 < plan.splits)))
+      (plan.splits > 1 && (!ws.slots || !ws.counters || !ws.tag || (ws.tag & kCountMask) ||
+                           plan.splits > kMaxSplits || g.K / 64 < plan.splits)))
     return hipErrorInvalidValue;
   block::BlockParams p{};
   p.A = static_cast<const uint16_t *>(g.A);
@@ -272,7 +297,7 @@ hipError_t launch_blocks(const GemmArgs &g, const GemmPlan &plan, const BlockWor
   p.splits = plan.splits;
   p.slots = ws.slots;
   p.counters = ws.counters;
-  p.epoch = ws.epoch;
+  p.tag = ws.tag;
   p.zero = ws.zero;
   p.zero_words = (uint32_t)ws.zero_words;
   const bool vec4 = rows_vec4(g);

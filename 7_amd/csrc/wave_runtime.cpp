@@ -9,8 +9,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <atomic>
-#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -426,19 +424,6 @@ int wave_gemm_streamk_noalloc_launch(const void *A, const void *B, void *C, int 
                                   counters, workers, stream);
 }
 
-// Launch epochs for counters that carry their launch's tag (the split-K
-// short-M kernel): process-wide, never 0, and started from the clock, so
-// that a workspace another process left behind is unlikely to hold one.
-static uint32_t next_epoch() {
-  static std::atomic<uint32_t> epoch{
-      (uint32_t)std::chrono::steady_clock::now().time_since_epoch().count()};
-  uint32_t e;
-  do
-    e = epoch.fetch_add(1u, std::memory_order_relaxed) + 1u;
-  while (e == 0u);
-  return e;
-}
-
 int wave_gemm_auto_workspace_bytes(int M, int N, int K, size_t *bytes) {
   if (!bytes)
     return fail(WAVE_ERR_INVALID, "gemm auto: null size output");
@@ -526,7 +511,7 @@ int wave_gemm_auto_launch(const void *A, const void *B, void *C, int M, int N, i
     if (plan.splits > 1) {
       ws.slots = static_cast<float *>(workspace);
       ws.counters = reinterpret_cast<unsigned long long *>(counter_base);
-      ws.epoch = next_epoch();
+      ws.tag = wave::gemm::split_tag();
     }
     if (have && short_m.splits > 0) {
       // Words no block counts on: the kernel clears them.

@@ -156,7 +156,8 @@ int wave_gemm_streamk_counters_check(const uint32_t *counters, int M, int N,
  * memory of wave_gemm_auto_workspace_bytes(M, N, K) bytes (0 when the shape
  * takes an unsplit path); it needs no initialisation: a Stream-K launch zeroes
  * the counters it uses with a fill kernel, and a split block's counters carry
- * a per-launch tag, so whatever they hold counts as zero.  For M <= 128 the
+ * a 60-bit tag drawn anew for each launch, so that what they held before counts
+ * as zero (but for a chance of 2^-60 a word).  For M <= 128 the
  * workspace ends in two 64-bit words per column block, which every launch
  * leaves zero.  With a smaller workspace an unsplit kernel runs.  One launch
  * in flight per workspace.  Same C as wave_gemm_launch (c_layout row- or

@@ -7,6 +7,7 @@ so every kernel, block size and K split has to give the oracle's bits.
 import pytest
 import torch
 
+import gemm_plan
 from conftest import to_dev
 from test_gemm_gpu import ODT, TDT, assert_exact, run_gemm
 
@@ -113,3 +114,21 @@ def test_split_graph_replays(wave, oracle, dev):
         torch.cuda.synchronize()
         assert_exact(oracle, out, ref, 0)
         assert_exact(oracle, other, ref1, 0)
+
+
+@pytest.mark.parametrize("shape", [(512, 512, 16384), (100, 5000, 12288)])
+def test_counter_words_of_other_launches(wave, oracle, dev, shape):
+    """Workspaces full of words that earlier launches left half counted: other
+    tags, with every count (both places where counters lie)."""
+    M, N, K = shape
+    a, b = oracle.gemm_inputs(M, K, 1, 27, 0), oracle.gemm_inputs(N, K, 1, 27, 1)
+    ref = oracle.gemm_nt(a, b, 1)
+    A, B = to_dev(a, TDT[1], dev), to_dev(b, TDT[1], dev)
+    need = wave.gemm_auto_workspace_bytes(M, N, K)
+    for count in range(16):
+        word = gemm_plan.split_tag(wave.runtime.lib()) | count
+        ws = torch.full((need // 8,), word - (1 << 64) * (word >> 63), dtype=torch.int64,
+                        device=dev).view(torch.uint8)
+        c = wave.gemm_auto(A, B, out_dtype="f32", workspace=ws)
+        torch.cuda.synchronize()
+        assert_exact(oracle, c, ref, 0)
