@@ -195,7 +195,8 @@ GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, int workers,
   const float hbm_mb = 2e-6f * (float)K * ((float)M + (float)N);
   for (const BlockCost &c : kBlocks) {
     const int64_t tiles = up(M, c.bm) * up(N, c.bn);
-    if (tiles > (1 << 24) || (!vec4 && (c.bm != 64 || c.bn != 64)))
+    // A grid holds fewer than 2^32 threads, 256 a block.
+    if (tiles >= (1 << 24) || (!vec4 && (c.bm != 64 || c.bn != 64)))
       continue;
     for (int splits = 1; splits <= (vec4 ? kMaxSplits : 1); ++splits) {
       if (splits > 1 &&

@@ -1,4 +1,7 @@
-"""Host side of the GEMM dispatch, without a GPU: the tags of split launches."""
+"""Host side of the GEMM dispatch, without a GPU: the tags of split launches and
+the kernel a shape takes."""
+
+import pytest
 
 import gemm_plan
 
@@ -15,3 +18,12 @@ def test_split_tags_are_drawn_from_sixty_bits(wave):
         assert abs(sum(t >> bit & 1 for t in tags) - 2048) < 400, bit
         flips = sum((a ^ b) >> bit & 1 for a, b in zip(tags, tags[1:]))
         assert abs(flips - 2048) < 400, bit
+
+
+@pytest.mark.parametrize("M,N,K", [(1 << 18, 1 << 18, 1), (1 << 18, 1 << 18, 5),
+                                   (1 << 24, 4096, 1), ((1 << 18) - 64, 1 << 18, 1),
+                                   (1 << 17, 1 << 17, 4), (1 << 28, 32, 4)])
+def test_block_grids_stay_below_2_32_threads(wave, M, N, K):
+    p = gemm_plan.plan(wave.runtime.lib(), M, N, K)
+    if p.bm:
+        assert -(-M // p.bm) * -(-N // p.bn) * p.splits * 256 < 1 << 32
