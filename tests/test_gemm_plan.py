@@ -4,6 +4,8 @@ the kernel a shape takes."""
 import pytest
 
 import gemm_plan
+from test_gemm_block_gpu import BLOCK_SHAPES, SPLIT_SHAPES, TILE_SHAPES, UNALIGNED_SHAPES
+from test_streamk_gpu import AUTO_SHAPES, auto_workers, short_m_plan
 
 
 def test_split_tags_are_drawn_from_sixty_bits(wave):
@@ -27,3 +29,37 @@ def test_block_grids_stay_below_2_32_threads(wave, M, N, K):
     p = gemm_plan.plan(wave.runtime.lib(), M, N, K)
     if p.bm:
         assert -(-M // p.bm) * -(-N // p.bn) * p.splits * 256 < 1 << 32
+
+
+# What the GPU tests' shapes take on 256 CUs, as their comments say.
+def test_block_shapes_take_every_block(wave):
+    lib = wave.runtime.lib()
+    plans = [gemm_plan.plan(lib, *s) for s in BLOCK_SHAPES]
+    assert {(p.bm, p.bn) for p in plans[:-2]} == {(32, 32), (32, 64), (64, 64), (128, 64),
+                                                  (128, 128)}
+    assert [p.bm for p in plans[-2:]] == [0, 0]
+    assert all((p.bm, p.bn) == (64, 64)
+               for p in (gemm_plan.plan(lib, *s) for s in UNALIGNED_SHAPES))
+    assert all(gemm_plan.plan(lib, M, N, K, vec4=K % 4 == 0 and off % 4 == 0).bm == 0
+               for M, N, K, off in TILE_SHAPES)
+
+
+def auto(lib, M, N, K):
+    return gemm_plan.auto_plan(lib, M, N, K, short_m_plan(M, N, K, 256),
+                               auto_workers(M, N, K, 256))
+
+
+def test_split_shapes_split_every_block(wave):
+    plans = [auto(wave.runtime.lib(), *s) for s in SPLIT_SHAPES]
+    assert all(p.splits > 1 for p in plans)
+    assert {(p.bm, p.bn) for p in plans} == {(32, 32), (32, 64), (64, 64), (128, 64), (128, 128)}
+    assert {p.splits for p in plans} >= {2, 3, 4, 5, 6, 8}
+
+
+def test_auto_shapes_take_what_they_name(wave):
+    lib = wave.runtime.lib()
+    for shape, kind in AUTO_SHAPES:
+        p = auto(lib, *shape)
+        got = ("stream-k" if p.workers else "tiles" if p.bm == 0 else
+               "split" if p.splits > 1 else "blocks")
+        assert got == kind, (shape, p)

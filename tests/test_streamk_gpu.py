@@ -196,23 +196,27 @@ def expected_workspace(wave, M, N, K, dev):
     return w, sb + cb
 
 
-@pytest.mark.parametrize("shape", [(2048, 512, 8192),    # 16 tiles, long K
-                                   (1000, 300, 4100),    # ragged, 8 tiles
-                                   # K % 4 != 0: the bounds-checked Stream-K kernel
-                                   (1000, 300, 4101),
-                                   # ragged, K off the stage, 16 tiles:
-                                   # 128 workers, 8-9 contributors a tile
-                                   (1000, 1000, 16400),
-                                   (4096, 4096, 512),    # 256 tiles
-                                   (3072, 3072, 8192),   # 144 tiles: uneven split
-                                   (4096, 2048, 4096),   # 128 tiles, K 4096
-                                   (128, 1024, 8192),    # split short-M kernel
-                                   (128, 1024, 192)])    # unsplit short-M kernel
+# What each takes on 256 CUs (test_gemm_plan.py): 256x256 tiles, blocks, blocks
+# with K split, or Stream-K.
+AUTO_SHAPES = [((2048, 512, 8192), "split"),     # 16 tiles, long K
+               ((1000, 300, 4100), "blocks"),    # ragged, 8 tiles
+               ((1000, 300, 4101), "blocks"),    # element by element
+               # K % 4 != 0, 20 tiles: the bounds-checked Stream-K kernel
+               ((1000, 1100, 16385), "stream-k"),
+               ((1000, 1000, 16400), "split"),   # ragged, K off the stage
+               ((4096, 4096, 512), "tiles"),     # 256 tiles
+               ((3072, 3072, 8192), "tiles"),    # 144 tiles
+               ((4096, 2048, 4096), "blocks"),   # 128 tiles, K 4096
+               ((128, 1024, 8192), "blocks"),    # M <= 128, with its workspace
+               ((128, 1024, 192), "blocks")]     # M <= 128, without
+
+
+@pytest.mark.parametrize("shape", [s for s, _ in AUTO_SHAPES])
 def test_auto_dispatch_matches_tiled(wave, oracle, dev, shape):
-    """The workspace size names the worker count the dispatch picks (checked
-    against the rules for this device's CU count).  Bucket inputs make every
-    sum exact, so the auto path (Stream-K or not) equals wave_gemm_launch bit
-    for bit; a too-small workspace falls back to the tiled kernel."""
+    """The workspace has the size of the worker count and the short-M slots that
+    the rules give for this device's CU count.  Bucket inputs make every sum
+    exact, so the auto path, whichever it is, equals wave_gemm_launch bit for
+    bit; a too-small workspace falls back to an unsplit kernel."""
     M, N, K = shape
     need = wave.gemm_auto_workspace_bytes(M, N, K)
     assert need == expected_workspace(wave, M, N, K, dev)[1]
