@@ -136,27 +136,36 @@ def test_auto_splits_bit_exact(wave, oracle, dev, in_dt, out_dt, layout, shape):
     assert bool((guard[need:] == 0xFF).all())
 
 
+# Both split on 256 CUs (test_gemm_plan.py); the second's partials reach to where
+# the first's counters lie (the top 32 KiB of 16 MiB).
+GRAPH_SHAPES = [(512, 512, 16384), (2048, 1024, 16384)]
+
+
 def test_split_graph_replays(wave, oracle, dev):
-    """A captured split launch (a fixed epoch) replayed between eager launches
-    of another shape on the same workspace."""
-    shapes = [(512, 512, 8192), (300, 260, 8260)]
+    """A captured split launch (a fixed tag) replayed between eager launches of
+    another shape on the same workspace, after the words it counts on were
+    written over, and twice in a row."""
     ops = []
-    for i, (M, N, K) in enumerate(shapes):
+    for i, (M, N, K) in enumerate(GRAPH_SHAPES):
         a, b = oracle.gemm_inputs(M, K, 1, 25 + i, 0), oracle.gemm_inputs(N, K, 1, 25 + i, 1)
         ops.append((to_dev(a, TDT[1], dev), to_dev(b, TDT[1], dev), oracle.gemm_nt(a, b, 1)))
-    need = max(wave.gemm_auto_workspace_bytes(*s) for s in shapes)
+    need = max(wave.gemm_auto_workspace_bytes(*s) for s in GRAPH_SHAPES)
     ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=dev)
     (A, B, ref), (A1, B1, ref1) = ops
     out = wave.gemm_auto(A, B, out_dtype="f32", workspace=ws)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         wave.gemm_auto(A, B, out_dtype="f32", workspace=ws, out=out)
-    for _ in range(4):
-        out.zero_()
+    noise = torch.randn(need // 4, device=dev).view(torch.uint8)
+    for i in range(4):
         other = wave.gemm_auto(A1, B1, out_dtype="f32", workspace=ws)
-        graph.replay()
-        torch.cuda.synchronize()
-        assert_exact(oracle, out, ref, 0)
+        if i & 1:
+            ws[:need // 4 * 4].copy_(noise)
+        for _ in range(2):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert_exact(oracle, out, ref, 0)
         assert_exact(oracle, other, ref1, 0)
 
 
