@@ -291,6 +291,16 @@ __host__ __device__ __forceinline__ int kv_items(int group, int nb, int kb2, boo
 __host__ __device__ __forceinline__ int kv_chunks(int items, int chunk) {
   return chunk > 0 ? (items + chunk - 1) / chunk : 1;
 }
+// The first item of chunk `index` of `count`: items * index / count rounded down,
+// whose product does not fit 32 bits where a block has millions of items (from 1.4
+// million query heads of 128 rows on one KV head on: Q, O, dO and dQ of 46 GB).
+__host__ __device__ constexpr int kv_first(int items, int index, int count) {
+  return items / count * index + items % count * index / count;
+}
+static_assert(kv_first(1 << 24, 700, 768) == (int)(((int64_t)1 << 24) * 700 / 768) &&
+                  kv_first(1 << 24, 768, 768) == 1 << 24 && kv_first(128, 2, 3) == 85 &&
+                  kv_first(5, 1, 3) == 1 && kv_first(5, 2, 3) == 3,
+              "chunk bounds");
 
 // CTA c (0 .. per_head-1) of a KV head -> its block, its chunk of the block's
 // items and how many the block has.
@@ -375,8 +385,8 @@ __global__ __launch_bounds__(512, 1) void bwd_kv_pp_kernel(BwdParams p) {
   // Work items (q head h, query block qb), h major; causal: the blocks at
   // or after group 0's key block (group 1's first one is wholly masked).
   const int qb0 = CAUSAL ? 2 * kb2 : 0, block_items = group * (nb - qb0);
-  const int first = block_items * chunk.index / chunk.count;
-  const int items = block_items * (chunk.index + 1) / chunk.count - first;
+  const int first = kv_first(block_items, chunk.index, chunk.count);
+  const int items = kv_first(block_items, chunk.index + 1, chunk.count) - first;
   struct Cursor {
     int h, qb;
   };
