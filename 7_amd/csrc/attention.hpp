@@ -46,6 +46,8 @@ struct BwdArgs {
   int cus = 256;               // compute units of the device
 };
 size_t bwd_workspace_bytes(int batch, int q_heads, int kv_heads, int seq, bool causal, int cus);
+// Keys a block of the dK/dV kernel that launch_bwd takes with its workspace: 64 or 128.
+int bwd_key_block(int batch, int q_heads, int kv_heads, int seq, bool causal, int cus);
 hipError_t launch_bwd(const BwdArgs &args, hipStream_t stream);
 
 // Block-scaled FP8 forward (attention_fwd8.hip): Q, K, V e4m3 bytes in the

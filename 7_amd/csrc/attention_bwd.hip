@@ -13,7 +13,7 @@
 // formulas above (oracle.py fa_backward) that is itself checked against
 // torch autograd.
 //
-// Three or four kernels, deterministic (no atomics):
+// Three or four kernels a call, deterministic (no atomics):
 //  * bwd_delta_kernel: -delta[row] = -sum_d dO[row][d] * O[row][d] in fp32
 //    (into the caller's scratch).
 //  * bwd_kv_pp_kernel: one CTA (8 waves, two groups of 4 one segment apart)
@@ -24,6 +24,9 @@
 //    registers.  Where those blocks are fewer than the CUs, or causal ones of
 //    uneven length, a block's loop is cut into chunks for several CTAs, which
 //    leave fp32 partials that bwd_kv_sum_kernel adds in chunk order.
+//    bwd_kv_kernel (one CTA of 4 waves per 64-key block, Q and dO staged through
+//    registers) takes over where half a block of 128 past the sequence costs more
+//    (half_blocks).
 //  * bwd_q_kernel: one CTA per 64-query block of one q head; it loops over
 //    the key blocks (causal: up to the diagonal) and accumulates dQ.
 // Every product is an "NT" product C[m][n] = sum_k A[m][k] B[n][k] of 32x32
@@ -36,11 +39,12 @@
 // between the score products and the gradient products.  LDS tiles are
 // unpadded with XOR-swizzled 16-byte chunks (swz below), conflict-free for
 // every read these kernels make: 130 KiB (bwd_kv_pp_kernel, one CTA per
-// CU) and 72 KiB (dQ) of LDS, two CTAs per CU.
+// CU), 48 KiB (bwd_kv_kernel) and 72 KiB (dQ) of LDS, two CTAs per CU.
 #include "attention.hpp"
 #include "wave_common.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace wave {
 namespace attention {
@@ -221,6 +225,33 @@ __device__ __forceinline__ void load_frags(const uint16_t *row, u32x4 (&f)[8]) {
     f[kk] = *reinterpret_cast<const u32x4 *>(row + 16 * kk + 8 * (lane >> 5));
 }
 
+// A [64][128] block of rows (row stride 128 elements) in flight through
+// registers: fetch() issues the global loads, put() writes the rows to LDS
+// (wide tile R).
+// Thread t handles row pairs x 16-byte chunks: unit u = t + 256*i, row pair
+// u / 16, chunk u % 16.
+struct BlockRegs {
+  u32x4 a[2], b[2];
+  __device__ __forceinline__ void fetch(const uint16_t *src) {
+    const uint32_t t = threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t u = t + 256u * i, rp = u >> 4, c = u & 15u;
+      a[i] = *reinterpret_cast<const u32x4 *>(src + (size_t)(2 * rp) * kBD + 8 * c);
+      b[i] = *reinterpret_cast<const u32x4 *>(src + (size_t)(2 * rp + 1) * kBD + 8 * c);
+    }
+  }
+  __device__ __forceinline__ void put(uint8_t *R) const {
+    const uint32_t t = threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t u = t + 256u * i, rp = u >> 4, c = u & 15u;
+      *reinterpret_cast<u32x4 *>(R + toff<256>(2 * rp, 16 * c)) = a[i];
+      *reinterpret_cast<u32x4 *>(R + toff<256>(2 * rp + 1, 16 * c)) = b[i];
+    }
+  }
+};
+
 // CTA id -> work index with the CTAs of one head on one XCD (the
 // dispatcher places workgroup i on XCD i % 8), so they share that head's
 // K/V or Q/dO rows in the XCD's L2.
@@ -283,6 +314,118 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(BwdParams p, int rows) {
     p.delta[row] = -s;
 }
 
+// dK, dV of one 64-key block of one KV head.
+template <int DT, bool CAUSAL>
+__global__ __launch_bounds__(256, 2) void bwd_kv_kernel(BwdParams p) {
+  __shared__ __attribute__((aligned(16))) uint8_t smem[2 * kWide + 2 * kNarrowS];
+  uint8_t *sQ = smem, *sdO = sQ + kWide, *sPt = sdO + kWide, *sdSt = sPt + kNarrowS;
+  const int nb = p.seq / kBlk;
+  int bhk, kb;
+  head_coords((int)blockIdx.x, p.batch * p.kv_heads, nb, 0, bhk, kb);
+  const int b = bhk / p.kv_heads, hkv = bhk - b * p.kv_heads;
+  const int group = p.q_heads / p.kv_heads;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const size_t kv_off = ((size_t)bhk * p.seq + (size_t)kb * kBlk) * kBD;
+
+  // Score tiles: wave w computes S[q][key] for q half w&1, key half w>>1;
+  // lane l holds key kh2*32 + l%32 and queries qh2*32 + 8g + 4(l/32) + e.
+  const int qh2 = wave & 1, kh2 = wave >> 1;
+  // Gradient tiles: key half w&1, d quarters 2(w>>1), 2(w>>1)+1.
+  const int kh = wave & 1, dq = wave >> 1;
+  // K and V rows of this wave's key half as B fragments, for the whole CTA.
+  u32x4 kf[8], vf[8];
+  load_frags(p.K + kv_off + (size_t)(kh2 * 32 + (lane & 31)) * kBD, kf);
+  load_frags(p.V + kv_off + (size_t)(kh2 * 32 + (lane & 31)) * kBD, vf);
+  // Gradient accumulators: dV columns (2 dq) * 32 and (2 dq + 1) * 32, then
+  // dK's.
+  f32x16 g[4] = {f32x16{}, f32x16{}, f32x16{}, f32x16{}};
+  const int key = kb * kBlk + kh2 * 32 + (int)(lane & 31);
+  // Work items: (q head h of the group, query block qb), h major (causal:
+  // the blocks at or after the key block); the next item's Q and dO rows
+  // and its lse / delta are fetched while this one's products run.
+  const int qb0 = CAUSAL ? kb : 0, items = group * (nb - qb0);
+  auto rows_of = [&](int h, int q) {  // first row of item (h, q) in [B*Hq*S]
+    return ((size_t)b * p.q_heads + (size_t)hkv * group + h) * p.seq + (size_t)q * kBlk;
+  };
+  // This wave's score rows of an item: lse and -delta of rows
+  // qh2*32 + 8 g + 4 (l / 32) + e as the accumulators' start values.
+  f32x16 s, dp;
+  auto load_stats = [&](size_t rb) {
+    const size_t r0 = rb + qh2 * 32 + 4 * (lane >> 5);
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      const f32x4 a = *reinterpret_cast<const f32x4 *>(p.lse + r0 + 8 * g4);
+      const f32x4 d = *reinterpret_cast<const f32x4 *>(p.delta + r0 + 8 * g4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[4 * g4 + e] = a[e];
+        dp[4 * g4 + e] = d[e];
+      }
+    }
+  };
+  int h = 0, qb = qb0;
+  BlockRegs rq, rdo;
+  rq.fetch(p.Q + rows_of(0, qb0) * kBD);
+  rdo.fetch(p.dO + rows_of(0, qb0) * kBD);
+  load_stats(rows_of(0, qb0));
+  for (int it = 0; it < items; ++it) {
+    int hn = h, qbn = qb + 1;
+    if (qbn == nb) {
+      qbn = qb0;
+      ++hn;
+    }
+    const bool more = it + 1 < items;
+    __syncthreads();  // the previous item's readers are done
+    rq.put(sQ);
+    rdo.put(sdO);
+    if (more) {
+      rq.fetch(p.Q + rows_of(hn, qbn) * kBD);
+      rdo.fetch(p.dO + rows_of(hn, qbn) * kBD);
+    }
+    // The score accumulator starts at -lse / scale and dP's at -delta, so
+    // exp2(c * s) = P and dp = dP - delta after the products.
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      s[r] *= -p.inv_scale;
+    __syncthreads();
+    mma2_nt_reg<DT>(s, sQ, kf, dp, sdO, vf, qh2 * 32);
+    // P and dS; P^T / dS^T rows = keys, 4 consecutive queries per store.
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4) {
+      float pv[4], dsv[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 4 * g4 + e;
+        const int q = qb * kBlk + qh2 * 32 + 8 * g4 + 4 * (int)(lane >> 5) + e;
+        float pr = __builtin_amdgcn_exp2f(s[r] * p.scale_log2);
+        if (CAUSAL && key > q)
+          pr = 0.f;
+        pv[e] = pr;
+        dsv[e] = pr * dp[r];
+      }
+      const uint32_t off =
+          toff<128>(kh2 * 32 + (lane & 31), 2 * (qh2 * 32 + 8 * g4 + 4 * (lane >> 5)));
+      *reinterpret_cast<u32x2 *>(sPt + off) = u32x2{pack2<DT>(pv[0], pv[1]), pack2<DT>(pv[2], pv[3])};
+      *reinterpret_cast<u32x2 *>(sdSt + off) =
+          u32x2{pack2<DT>(dsv[0], dsv[1]), pack2<DT>(dsv[2], dsv[3])};
+    }
+    __syncthreads();
+    const uint8_t *const ga[2] = {sPt, sdSt};
+    const uint8_t *const gr[2] = {sdO, sQ};
+    mma_grad<DT, 2>(g, ga, kh * 32, gr, (2 * dq) * 32, (2 * dq + 1) * 32);
+    if (more)
+      load_stats(rows_of(hn, qbn));
+    h = hn;
+    qb = qbn;
+  }
+  uint16_t *dK = p.dK + kv_off, *dV = p.dV + kv_off;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    store_tile32<DT>(dV, kh * 32, (2 * dq + t) * 32, g[t], 1.f);
+    store_tile32<DT>(dK, kh * 32, (2 * dq + t) * 32, g[2 + t], p.scale);
+  }
+}
+
 // Work items of 128-key block kb2 of a KV head: (q head of the group, 64-query
 // block); causal: the blocks at or after the key block.
 __host__ __device__ __forceinline__ int kv_items(int group, int nb, int kb2, bool causal) {
@@ -322,7 +465,8 @@ __device__ __forceinline__ KvChunk kv_chunk(const BwdParams &p, int group, int n
 }
 
 // dK, dV of a 128-key block of one KV head as two groups of four waves:
-// group g (waves 4g .. 4g+3) owns keys 64 g .. 64 g + 63 of the block, on
+// group g (waves 4g .. 4g+3) owns keys 64 g .. 64 g + 63 of the block and
+// does for them what bwd_kv_kernel does for its 64 keys (the same products), on
 // the same work items.  The groups share each item's Q
 // and dO rows and its rows' lse and -delta, which arrive by LDS DMA into a
 // 3-buffer ring (so no global load is waited for inside the loop), and run
@@ -656,8 +800,42 @@ namespace {
 // The dK/dV kernel's split: the chunk length and the CTAs a KV head then has.
 struct KvPlan {
   int chunk = 0, per_head = 0;
-  bool sum = false;  // some block has several chunks
+  bool sum = false;   // some block has several chunks
+  bool half = false;  // bwd_kv_kernel's 64-key blocks
 };
+
+// Whether bwd_kv_kernel's 64-key blocks are the faster whole blocks of an odd
+// number nb of them.  128-key blocks spend half of the last one on keys past the
+// sequence, one CTA a CU; 64-key ones run two a CU, with more LDS traffic an item.
+// us a CTA to start and end, and an item, fitted to 130 measured shapes: 3.6 (3.3
+// in many rounds) and 1.75; 1.1 and 2.07 (alone on its CU), 2.85 and 2.5 (two a CU).  Causal blocks by
+// length end level (0.86, but the longest come in whole rounds); head by head, two
+// or four lengths in turn fall on the same CUs each time (1.25 over many rounds).
+// The backward (us, 128-key / 64-key): S64 B32 H16 32.9 / 26.3, B256 H16 247 / 208,
+// B1 H8 15.5 / 13.8, Hq64 Hkv1 130 / 154; S192 B24 H12 62.5 / 54.5, B128 Hq16 Hkv2
+// 254 / 282; S320 B32 H16 180 / 188; causal S448 B64 H16 534 / 488, S960 B32 H16 745
+// / 758.
+bool half_blocks(int64_t heads, int group, int nb, bool causal, bool by_length, int cus) {
+  const int nkb = (nb + 1) / 2;
+  const double longest = (double)group * nb, mean = (double)group * nkb;  // causal: of a block
+  const double n128 = (double)heads * nkb, n64 = (double)heads * nb;      // CTAs
+  const double one128 = 3.6 + 1.75 * longest, one64 = 1.1 + 2.07 * longest,
+               two64 = 2.85 + 2.5 * longest;
+  double t128, t64;
+  if (causal && nb > 1) {
+    const double turns = by_length ? 0.86
+                         : (nkb == 2 || nkb == 4) && n128 >= 8 * cus ? 1.25
+                                                                     : 1.0;
+    t128 = std::max(one128 * (by_length ? std::ceil((double)heads / cus) : 1.0),
+                    n128 > cus ? turns * (3.3 + 1.75 * mean) * n128 / cus : 0.0);
+    t64 = n64 <= cus ? one64 : std::max(two64, (2.85 + 2.5 * mean) * n64 / (2 * cus));
+  } else {
+    const double rounds = std::floor(n64 / (2 * cus)), rest = n64 - rounds * 2 * cus;
+    t128 = one128 * std::ceil(n128 / cus);
+    t64 = rounds * two64 + (rest == 0 ? 0.0 : rest <= cus ? one64 : two64);
+  }
+  return t64 < t128;
+}
 
 // A CTA takes 1.75 us an item (measured) and 4 to start and end; a CU runs one
 // at a time.  Splitting adds the sum kernel: 4 us and 0.06 a CTA (its 128 KiB
@@ -671,7 +849,9 @@ struct KvPlan {
 // blocks of one CTA each.  B2 Hq32 Hkv8 S4096 (512 blocks, two a CU): whole by
 // length 1014, chunks 1156, whole head by head 1051 for the whole backward; S2048
 // (256 blocks): whole 358, chunks 308.
-KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, bool by_length, int cus) {
+// split: with the chunks among the candidates.
+KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, bool by_length, int cus,
+               bool split) {
   const int64_t heads = (int64_t)batch * kv_heads;
   const int nkb = (nb + 1) / 2, longest = group * nb;
   auto per_head = [&](int chunk) {
@@ -693,7 +873,7 @@ KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, bool by_
   plan.per_head = nkb;
   double best = by_length ? 4 + 1.75 * std::max((double)longest, (double)total * heads / cus + 2)
                           : time(heads * nkb, longest);
-  for (int rounds = 1; rounds <= 3; ++rounds) {
+  for (int rounds = 1; split && rounds <= 3; ++rounds) {
     const int64_t most = (int64_t)rounds * cus / heads;
     if (most <= nkb)
       continue;
@@ -716,20 +896,27 @@ KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, bool by_
       plan.sum = true;
     }
   }
+  if (!plan.sum && nb % 2 && half_blocks(heads, group, nb, causal, by_length, cus)) {
+    plan.half = true;
+    plan.per_head = nb;
+  }
   return plan;
 }
 
 constexpr size_t kPartBytes = 16 * 512 * sizeof(f32x4);  // a CTA's dK, dV in fp32
 
 template <int DT, bool CAUSAL>
-hipError_t launch_bwd_dt(const BwdParams &p, bool sum, hipStream_t stream) {
+hipError_t launch_bwd_dt(const BwdParams &p, const KvPlan &plan, hipStream_t stream) {
   const int rows = p.batch * p.q_heads * p.seq;
   hipLaunchKernelGGL((bwd_delta_kernel<DT>), dim3((rows + 15) / 16), dim3(256), 0, stream, p,
                      rows);
   const int nb = p.seq / kBlk, heads = p.batch * p.kv_heads;
-  hipLaunchKernelGGL((bwd_kv_pp_kernel<DT, CAUSAL>), dim3(p.per_head * heads), dim3(512), 0, stream,
-                     p);
-  if (sum)
+  if (plan.half)
+    hipLaunchKernelGGL((bwd_kv_kernel<DT, CAUSAL>), dim3(nb * heads), dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL((bwd_kv_pp_kernel<DT, CAUSAL>), dim3(p.per_head * heads), dim3(512), 0,
+                       stream, p);
+  if (plan.sum)
     hipLaunchKernelGGL((bwd_kv_sum_kernel<DT, CAUSAL>), dim3((nb + 1) / 2 * heads * 4), dim3(512),
                        0, stream, p);
   hipLaunchKernelGGL((bwd_q_kernel<DT, CAUSAL>), dim3(nb * p.batch * p.q_heads), dim3(256), 0,
@@ -753,8 +940,14 @@ bool kv_order(int batch, int q_heads, int kv_heads, int seq, bool causal) {
 
 size_t bwd_workspace_bytes(int batch, int q_heads, int kv_heads, int seq, bool causal, int cus) {
   const KvPlan plan = kv_plan(batch, kv_heads, q_heads / kv_heads, seq / kBlk, causal,
-                              kv_order(batch, q_heads, kv_heads, seq, causal), cus);
+                              kv_order(batch, q_heads, kv_heads, seq, causal), cus, true);
   return plan.sum ? (size_t)batch * kv_heads * plan.per_head * kPartBytes : 0;
+}
+
+int bwd_key_block(int batch, int q_heads, int kv_heads, int seq, bool causal, int cus) {
+  const KvPlan plan = kv_plan(batch, kv_heads, q_heads / kv_heads, seq / kBlk, causal,
+                              kv_order(batch, q_heads, kv_heads, seq, causal), cus, true);
+  return plan.half ? kBlk : 2 * kBlk;
 }
 
 hipError_t launch_bwd(const BwdArgs &a, hipStream_t stream) {
@@ -777,14 +970,14 @@ hipError_t launch_bwd(const BwdArgs &a, hipStream_t stream) {
   p.scale = a.scale > 0.f ? a.scale : 1.0f / __builtin_sqrtf((float)kBD);
   p.scale_log2 = p.scale * kLog2eB;
   p.inv_scale = 1.0f / p.scale;
+  const int group = a.q_heads / a.kv_heads, nb = a.seq / kBlk;
   const bool kv_whole_order = kv_order(a.batch, a.q_heads, a.kv_heads, a.seq, a.causal != 0);
-  KvPlan plan = kv_plan(a.batch, a.kv_heads, a.q_heads / a.kv_heads, a.seq / kBlk, a.causal != 0,
-                        kv_whole_order, a.cus);
-  if (plan.sum && (!a.workspace || a.workspace_bytes < (size_t)a.batch * a.kv_heads *
-                                                           plan.per_head * kPartBytes)) {
-    plan = KvPlan{};
-    plan.per_head = (a.seq / kBlk + 1) / 2;
-  }
+  auto plan_for = [&](bool split) {
+    return kv_plan(a.batch, a.kv_heads, group, nb, a.causal != 0, kv_whole_order, a.cus, split);
+  };
+  KvPlan plan = plan_for(a.workspace != nullptr);
+  if (plan.sum && a.workspace_bytes < (size_t)a.batch * a.kv_heads * plan.per_head * kPartBytes)
+    plan = plan_for(false);
   p.chunk = plan.chunk;
   p.per_head = plan.per_head;
   p.part = static_cast<f32x4 *>(a.workspace);
@@ -792,10 +985,10 @@ hipError_t launch_bwd(const BwdArgs &a, hipStream_t stream) {
   p.q_by_length = by_length((int64_t)a.batch * a.q_heads, (int64_t)a.batch * a.kv_heads, a.seq,
                             a.causal != 0);
   if (a.dtype == kF16)
-    return a.causal ? launch_bwd_dt<kF16, true>(p, plan.sum, stream)
-                    : launch_bwd_dt<kF16, false>(p, plan.sum, stream);
-  return a.causal ? launch_bwd_dt<kBF16, true>(p, plan.sum, stream)
-                  : launch_bwd_dt<kBF16, false>(p, plan.sum, stream);
+    return a.causal ? launch_bwd_dt<kF16, true>(p, plan, stream)
+                    : launch_bwd_dt<kF16, false>(p, plan, stream);
+  return a.causal ? launch_bwd_dt<kBF16, true>(p, plan, stream)
+                  : launch_bwd_dt<kBF16, false>(p, plan, stream);
 }
 
 } // namespace attention

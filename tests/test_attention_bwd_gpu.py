@@ -51,10 +51,25 @@ def check(got, ref, dt):
 @pytest.mark.parametrize("dt", [1, 2])
 @pytest.mark.parametrize("causal", [False, True])
 # S % 128 == 0 runs the two-group dK/dV kernel (several 128-key blocks, GQA
-# and causal at 384), the other lengths the 64-key one.
+# and causal at 384), the other lengths that one or the 64-key one
+# (test_bwd_plan.py).
 @pytest.mark.parametrize("B,Hq,Hkv,S", [(1, 2, 2, 64), (1, 2, 2, 256), (2, 4, 2, 192),
                                          (1, 4, 1, 320), (2, 4, 2, 384)])
 def test_fa_bwd_parity(wave, oracle, dev, dt, causal, B, Hq, Hkv, S):
+    got, ref = run_bwd(wave, oracle, dev, dt, B, Hq, Hkv, S, causal)
+    check(got, ref, dt)
+
+
+# Odd numbers of 64-row blocks that take 64-key dK/dV blocks on 256 CUs
+# (test_bwd_plan.py): alone on their CUs, two a CU, and over several rounds.
+HALF_SHAPES = [(1, 8, 8, 64), (20, 8, 8, 64), (2, 12, 6, 64), (1, 5, 5, 192), (24, 12, 12, 192),
+               (1, 8, 8, 320), (90, 8, 8, 64)]
+
+
+@pytest.mark.parametrize("dt", [1, 2])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,S", HALF_SHAPES)
+def test_fa_bwd_half_blocks(wave, oracle, dev, dt, causal, B, Hq, Hkv, S):
     got, ref = run_bwd(wave, oracle, dev, dt, B, Hq, Hkv, S, causal)
     check(got, ref, dt)
 
