@@ -982,8 +982,13 @@ hipError_t launch_bwd(const BwdArgs &a, hipStream_t stream) {
   p.per_head = plan.per_head;
   p.part = static_cast<f32x4 *>(a.workspace);
   p.kv_by_length = kv_whole_order && !plan.sum;
+  // Two or three query blocks a head on more than one round (two CTAs a CU) have
+  // little to level and read K and V once more each: head by head -> by length, the
+  // backward, B64 H16 S192 168.8 -> 171.7, B32 H16 S192 88 -> 92, B128 Hq32 Hkv8 S128
+  // 283 -> 287; within a round B8 Hq16 Hkv4 S192 43.3 -> 41.7.
   p.q_by_length = by_length((int64_t)a.batch * a.q_heads, (int64_t)a.batch * a.kv_heads, a.seq,
-                            a.causal != 0);
+                            a.causal != 0) &&
+                  (nb >= 4 || (int64_t)nb * a.batch * a.q_heads <= 2 * a.cus);
   if (a.dtype == kF16)
     return a.causal ? launch_bwd_dt<kF16, true>(p, plan, stream)
                     : launch_bwd_dt<kF16, false>(p, plan, stream);
