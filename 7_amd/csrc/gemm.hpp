@@ -54,11 +54,13 @@ struct GemmPlan {
 struct SplitLimits {
   size_t slot_bytes = 0, counter_words = 0;
 };
-// vec4: K % 4 == 0 and A, B 8-byte aligned; workers: what Stream-K would run
-// with (0: not offered).
-GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, int workers,
+// vec4: K % 4 == 0 and A, B 8-byte aligned (rows_vec4); c_vec: C's lines start at
+// multiples of 16 bytes (lines_vec16); workers: what Stream-K would run with (0: not
+// offered).
+GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, bool c_vec, int workers,
                    const SplitLimits &limits);
 bool rows_vec4(const GemmArgs &args);
+bool lines_vec16(const GemmArgs &args);
 // A small-block launch: `slots` / `counters` for splits > 1 (any contents: a
 // counter word counts only under this launch's `tag`; left zero),
 // and zero_words 64-bit words at `zero` left zero.

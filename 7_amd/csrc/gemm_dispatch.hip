@@ -108,6 +108,10 @@ int k_iterations(int K) { return (K + kSKUnit - 1) / kSKUnit; }
 bool rows_vec4(const GemmArgs &g) {
   return g.K % 4 == 0 && aligned_to(g.A, 8) && aligned_to(g.B, 8);
 }
+bool lines_vec16(const GemmArgs &g) {
+  const size_t line = (size_t)(g.col_major ? g.M : g.N) * (g.out_dtype == kF32 ? 4 : 2);
+  return aligned_to(g.C, 16) && line % 16 == 0;
+}
 
 // ---- which kernel a shape takes --------------------------------------------
 // Each candidate's time is estimated (microseconds) and the least taken.  The
@@ -141,19 +145,32 @@ constexpr BlockCost kBlocks[] = {
 // Rows off 8 bytes (element-by-element loads through registers): a stage of
 // the 256x256 kernel, and of a 64x64 block alone on its CU or sharing it with
 // others (1000^2 x 1001 60.3 us in tiles, 15.8 in blocks; 2048^2 59.8 / 32.7;
-// 3000^2 62.8 / about 70).
-constexpr float kMaskedTile = 3.4f, kMaskedBlock = .8f, kMaskedShared = .46f;
+// 3000^2 62.8 / about 70).  Short K: storing C counts, a round of tiles 23.5 us
+// without its stages, of blocks 2.7 a CTA (10.3 and 1.6 where C's lines start at 16
+// bytes).  us, tiles / blocks: 4293 x 7657 x 51 62 / 91, 2472 x 4628 x 23 30.0 /
+// 38.4, 1450 x 7431 x 87 31 / 41, 1872 x 2891 x 21 24.6 / 19.6, 1141 x 4300 x 215
+// 34.5 / 26.9, 7038 x 664 x 43 13.6 / 11.8.
+constexpr float kMaskedTile = 3.35f, kMaskedBlock = .8f, kMaskedShared = .46f;
+constexpr float kMaskedTileStore[2] = {23.5f, 10.3f}, kMaskedBlockStore[2] = {2.7f, 1.6f};
 constexpr int kMinSplitStages = 4;  // stages a split keeps
+// Operands that the 256 MB last-level cache does not hold, with rows off its lines:
+// blocks on more than one round fetch their panels, shared lines and all, again and
+// again from HBM.  f16 us, tiles / 64x64 blocks: 5421 x 905 x 18996 (240 MB) 519 /
+// 578, 1332 x 3665 x 36640 839 / 993, 627 x 7008 x 37280 865 / 988; 128x64 ones: 2982
+// x 1372 x 35408 902 / 976, 1402 x 3089 x 33568 749 / 800.  Below, 2319 x 1678 x 22072
+// (176 MB) 592 / 503; whole lines, 1937 x 2465 x 27840 (245 MB) 570 / 548.
+constexpr float kFarMB = 235.f, kFarStage = 1.25f;
 
 int64_t up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // The cube of a block launch's estimate (the smooth maximum of its own time
 // and its operands' time from HBM, without the root).
 float block_cost3(const BlockCost &c, int64_t tiles, int64_t nk, int splits, int cus,
-                  float hbm_mb) {
+                  float hbm_mb, bool off_lines) {
   const int64_t ctas = tiles * splits, stages = up(nk, splits), load = up(ctas, cus);
+  const bool far = off_lines && hbm_mb > kFarMB;
   const float stage = ctas <= cus ? c.s0 + (c.s1 - c.s0) * (float)ctas / (float)cus
-                                  : c.s2 * (float)load;
+                                  : c.s2 * (float)load * (far ? kFarStage : 1.f);
   float t = c.base + stage * (float)stages + (float)(load - 1) * c.round;
   if (splits > 1)
     t += c.e0 + c.e1 * (float)(ctas * (c.bm * c.bn)) * 4e-6f +
@@ -171,7 +188,7 @@ float tile_stage(float busy, bool vec4) {
 float cube(float t) { return t * t * t; }
 } // namespace
 
-GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, int workers,
+GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, bool c_vec, int workers,
                    const SplitLimits &limits) {
   GemmPlan plan;
   // Block row and column numbers are ints with room for a block's edge; far
@@ -180,8 +197,10 @@ GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, int workers,
     return plan;
   const int64_t nk = up(K, 64), big = up(M, 256) * up(N, 256), rounds = up(big, cus);
   const bool ragged = M % 256 || N % 256 || K % 64;
-  float best = cube(7.f + (float)rounds * tile_stage((float)big / (float)(rounds * cus), vec4) *
-                              (float)nk + (float)(rounds - 1) * 4.f + (ragged ? 3.f : 0.f));
+  float best =
+      vec4 ? cube(7.f + (float)rounds * tile_stage((float)big / (float)(rounds * cus), true) *
+                            (float)nk + (float)(rounds - 1) * 4.f + (ragged ? 3.f : 0.f))
+           : cube(1.f + (float)rounds * (kMaskedTileStore[c_vec] + kMaskedTile * (float)nk));
   if (workers > 0) {
     // Stream-K: a worker's share of the stages, and 32 for the counter fill,
     // the publish and the reduction.
@@ -205,9 +224,10 @@ GemmPlan gemm_plan(int M, int N, int K, int cus, bool vec4, int workers,
            (size_t)tiles * 2 > limits.counter_words))
         break;
       const float t =
-          vec4 ? block_cost3(c, tiles, nk, splits, cus, hbm_mb)
-               : cube(c.base + (float)nk * std::max(kMaskedBlock,
-                                                    kMaskedShared * (float)up(tiles, cus)));
+          vec4 ? block_cost3(c, tiles, nk, splits, cus, hbm_mb, K % 64 != 0)
+               : cube(c.base +
+                      (float)nk * std::max(kMaskedBlock, kMaskedShared * (float)up(tiles, cus)) +
+                      (float)(up(tiles, cus) - 1) * kMaskedBlockStore[c_vec]);
       if (t < best) {
         best = t;
         plan.bm = c.bm;
@@ -294,7 +314,7 @@ hipError_t launch_blocks(const GemmArgs &g, const GemmPlan &plan, const BlockWor
   p.N = g.N;
   p.K = g.K;
   p.ldc = g.col_major ? g.M : g.N;
-  p.c_vec_ok = aligned_to(g.C, 16) && (size_t)p.ldc * (g.out_dtype == kF32 ? 4 : 2) % 16 == 0;
+  p.c_vec_ok = lines_vec16(g);
   p.splits = plan.splits;
   p.slots = ws.slots;
   p.counters = ws.counters;
@@ -317,7 +337,8 @@ hipError_t launch_blocks(const GemmArgs &g, const GemmPlan &plan, const BlockWor
 
 hipError_t launch(const GemmArgs &g, hipStream_t stream) {
   if (g.workers == 0 && !g.force_masked && !g.packed) {
-    const GemmPlan plan = gemm_plan(g.M, g.N, g.K, g.cus, rows_vec4(g), 0, SplitLimits{});
+    const GemmPlan plan = gemm_plan(g.M, g.N, g.K, g.cus, rows_vec4(g), lines_vec16(g), 0,
+                                    SplitLimits{});
     if (plan.bm)
       return launch_blocks(g, plan, BlockWorkspace{}, stream);
   }

@@ -505,7 +505,8 @@ int wave_gemm_auto_launch(const void *A, const void *B, void *C, int M, int N, i
     counter_base -= kWords * sizeof(uint64_t);
   }
   const wave::gemm::GemmPlan plan =
-      wave::gemm::gemm_plan(M, N, K, cus, wave::gemm::rows_vec4(g), workers, limits);
+      wave::gemm::gemm_plan(M, N, K, cus, wave::gemm::rows_vec4(g), wave::gemm::lines_vec16(g),
+                            workers, limits);
   if (plan.bm) {
     wave::gemm::BlockWorkspace ws;
     if (plan.splits > 1) {

@@ -25,13 +25,17 @@ def split_tag(lib):
     return fn()
 
 
-def plan(lib, M, N, K, cus=256, vec4=None, workers=0, slot_bytes=0, counter_words=0):
-    """What wave_gemm_launch runs (no workspace limits given)."""
-    fn = lib._ZN4wave4gemm9gemm_planEiiiibiRKNS0_11SplitLimitsE
+def plan(lib, M, N, K, cus=256, vec4=None, workers=0, slot_bytes=0, counter_words=0,
+         c_vec=None):
+    """What wave_gemm_launch runs (no workspace limits given); c_vec: by default
+    that of a 16-bit row-major C."""
+    fn = lib._ZN4wave4gemm9gemm_planEiiiibbiRKNS0_11SplitLimitsE
     fn.restype = Plan
-    fn.argtypes = [ctypes.c_int] * 4 + [ctypes.c_bool, ctypes.c_int, ctypes.POINTER(_Limits)]
+    fn.argtypes = [ctypes.c_int] * 4 + [ctypes.c_bool] * 2 + [ctypes.c_int,
+                                                              ctypes.POINTER(_Limits)]
     limits = _Limits(slot_bytes, counter_words)
-    return fn(M, N, K, cus, K % 4 == 0 if vec4 is None else vec4, workers, ctypes.byref(limits))
+    return fn(M, N, K, cus, K % 4 == 0 if vec4 is None else vec4,
+              N % 8 == 0 if c_vec is None else c_vec, workers, ctypes.byref(limits))
 
 
 def auto_plan(lib, M, N, K, short_m, workers, cus=256):

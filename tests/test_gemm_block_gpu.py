@@ -36,9 +36,10 @@ def test_blocks_bit_exact(wave, oracle, dev, in_dt, out_dt, layout, shape):
     assert_exact(oracle, c, ref, out_dt)
 
 
-# K not a multiple of 4: element-by-element loads, 64x64 blocks.
+# K not a multiple of 4: element-by-element loads, 64x64 blocks, and for the last
+# two shapes (short K, many blocks) the 256x256 tiles (test_gemm_plan.py).
 UNALIGNED_SHAPES = [(1, 1, 1), (64, 64, 63), (65, 129, 65), (200, 300, 130),
-                    (1000, 70, 1001), (3000, 3000, 65)]
+                    (1000, 70, 1001), (1872, 891, 21), (3000, 3000, 65), (1450, 7431, 87)]
 
 
 @pytest.mark.parametrize("layout,out_dt", [("row", 2), ("col", 0)])

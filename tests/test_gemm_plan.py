@@ -39,10 +39,30 @@ def test_block_shapes_take_every_block(wave):
     assert {(p.bm, p.bn) for p in plans[:-2]} == {(32, 32), (32, 64), (64, 64), (128, 64),
                                                   (128, 128)}
     assert [p.bm for p in plans[-2:]] == [0, 0]
-    assert all((p.bm, p.bn) == (64, 64)
-               for p in (gemm_plan.plan(lib, *s) for s in UNALIGNED_SHAPES))
+    plans = [gemm_plan.plan(lib, *s) for s in UNALIGNED_SHAPES]
+    assert all((p.bm, p.bn) == (64, 64) for p in plans[:-2])
+    assert [p.bm for p in plans[-2:]] == [0, 0]
     assert all(gemm_plan.plan(lib, M, N, K, vec4=K % 4 == 0 and off % 4 == 0).bm == 0
                for M, N, K, off in TILE_SHAPES)
+
+
+# (M, N, K, block): the faster kernel as measured, element by element.
+@pytest.mark.parametrize("M,N,K,bm", [
+    (4293, 7657, 51, 0), (2472, 4628, 23, 0), (1927, 7182, 49, 0), (2758, 7945, 11, 0),
+    (6651, 1032, 311, 0), (3000, 3000, 1001, 0), (1872, 2891, 21, 64), (1141, 4300, 215, 64),
+    (7038, 664, 43, 64), (2007, 1464, 4845, 64), (2048, 2048, 1001, 64), (1000, 1000, 1001, 64)])
+def test_unaligned_rows_by_shape(wave, M, N, K, bm):
+    assert gemm_plan.plan(wave.runtime.lib(), M, N, K).bm == bm
+
+
+# Operands beyond the last-level cache: no 64x64 blocks in several rounds where
+# rows lie off its lines.
+@pytest.mark.parametrize("M,N,K,bm", [
+    (5421, 905, 18996, 0), (1332, 3665, 36640, 0), (627, 7008, 37280, 0), (746, 6165, 34196, 0),
+    (1553, 2621, 36652, 0), (1121, 4345, 26000, 0), (2319, 1678, 22072, 64),
+    (1937, 2465, 27840, 64), (2539, 1669, 17440, 64)])
+def test_long_k_by_shape(wave, M, N, K, bm):
+    assert gemm_plan.plan(wave.runtime.lib(), M, N, K).bm == bm
 
 
 def auto(lib, M, N, K):
