@@ -92,6 +92,12 @@ template <int BM_, int BN_> struct BlockCfg {
   static constexpr int AI = BM / 32, BI = BN / 32;      // DMA issues per wave a stage
   static constexpr int DMA = AI + BI;
   static constexpr int SLOT = BM * BN;                  // floats per partial slot
+  // Up to SHORT stages go without the ring, whose other slots would be filled for
+  // nothing: 1 x 6976 x 64 3.32 -> 3.12 us (rocprofv3), 64 x 5696 x 128 3.64 -> 3.40,
+  // 32 x 4096 x 256 3.72 -> 3.36; 1536 x 2048 x 256 in blocks of 128x128 6.92 -> 7.16,
+  // so two stages there.
+  static constexpr int SHORT = OCC == 2 ? 4 : 2;
+  static_assert(SHORT <= NS, "a slot a stage");
   static_assert(DMA * (NS - 2) < 64, "vmcnt budget");
 };
 
@@ -272,46 +278,58 @@ __global__ __launch_bounds__(256, X::OCC) void block_kernel(BlockParams p) {
           dma16(l + X::AB + (wave * X::BI + d - X::AI) * 1024, b0 + at, gob[d - X::AI] & keep);
       };
       asm volatile("" ::: "memory");  // the remainder's loads stay ahead of the DMA
-#pragma unroll
-      for (int s = 0; s < NS; ++s)
-#pragma unroll
-        for (int d = 0; d < X::DMA; ++d)
-          issue1(s, s, d);
-      vm_wait_barrier<X::DMA *(NS - 1)>();
-      // Stage k from registers, stage k + 1 read into the other set and stage
-      // k + NS issued into stage k's slot, spread over the MFMAs (the reads
-      // over the first three quarters, so that the next barrier finds them
-      // done).
-      constexpr int RM = NM * 3 / 4 > 0 ? NM * 3 / 4 : 1;
-      int s = 0;
-      auto step = [&](const Frag &cur, Frag &nxt, int k) {
-        // Stage k + 1 has landed (stages k + 2 .. k + NS - 1 may be in
-        // flight) and every wave holds stage k in registers.
-        vm_wait_barrier<X::DMA *(NS - 2)>();
-        const int free_slot = s;
-        s = s == NS - 1 ? 0 : s + 1;
-        multiply(cur, [&](int m) {
-#pragma unroll
-          for (int r = 0; r < NR; ++r)
-            if (r * RM / NR == m)
-              read1(nxt, s, r);
+      if (len <= X::SHORT) {
+        // A few stages: no ring to fill behind them.
+        for (int s = 0; s < len; ++s)
 #pragma unroll
           for (int d = 0; d < X::DMA; ++d)
-            if (d * NM / X::DMA == m)
-              issue1(free_slot, k + NS, d);
-          __builtin_amdgcn_sched_barrier(0);
-        });
-      };
-      Frag f[2];
-      read(f[0], 0);
-      int k = 0;
-      for (; k + 1 < len; k += 2) {
-        step(f[0], f[1], k);
-        step(f[1], f[0], k + 1);  // past the last stage the reads go unused
+            issue1(s, s, d);
+        vm_wait_barrier();
+        for (int s = 0; s < len; ++s)
+          whole_stage(s);
+        lds_barrier();  // every wave is done with the ring
+      } else {
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+          for (int d = 0; d < X::DMA; ++d)
+            issue1(s, s, d);
+        vm_wait_barrier<X::DMA *(NS - 1)>();
+        // Stage k from registers, stage k + 1 read into the other set and stage
+        // k + NS issued into stage k's slot, spread over the MFMAs (the reads
+        // over the first three quarters, so that the next barrier finds them
+        // done).
+        constexpr int RM = NM * 3 / 4 > 0 ? NM * 3 / 4 : 1;
+        int s = 0;
+        auto step = [&](const Frag &cur, Frag &nxt, int k) {
+          // Stage k + 1 has landed (stages k + 2 .. k + NS - 1 may be in
+          // flight) and every wave holds stage k in registers.
+          vm_wait_barrier<X::DMA *(NS - 2)>();
+          const int free_slot = s;
+          s = s == NS - 1 ? 0 : s + 1;
+          multiply(cur, [&](int m) {
+#pragma unroll
+            for (int r = 0; r < NR; ++r)
+              if (r * RM / NR == m)
+                read1(nxt, s, r);
+#pragma unroll
+            for (int d = 0; d < X::DMA; ++d)
+              if (d * NM / X::DMA == m)
+                issue1(free_slot, k + NS, d);
+            __builtin_amdgcn_sched_barrier(0);
+          });
+        };
+        Frag f[2];
+        read(f[0], 0);
+        int k = 0;
+        for (; k + 1 < len; k += 2) {
+          step(f[0], f[1], k);
+          step(f[1], f[0], k + 1);  // past the last stage the reads go unused
+        }
+        if (k < len)
+          multiply(f[0], [](int) {});
+        vm_wait_barrier();  // the DMA past the end, before the ring is written again
       }
-      if (k < len)
-        multiply(f[0], [](int) {});
-      vm_wait_barrier();  // the DMA past the end, before the ring is written again
     }
     if (tail) {
       store_regs(0);

@@ -24,6 +24,7 @@ BLOCK_SHAPES = [
     (500, 300, 1100), (515, 1021, 64), (400, 1600, 260), (1000, 1000, 132),
     (1024, 1536, 192), (1290, 1270, 72), (129, 8192, 324),                  # 64 and 128 edges
     (1536, 2048, 256), (2000, 1500, 100), (16400, 256, 64),
+    (64, 96, 256), (64, 96, 320), (1536, 2048, 128), (1536, 2048, 192),     # with and without ring
     (3000, 3000, 132), (3072, 3300, 64)]
 
 
