@@ -47,10 +47,15 @@ hipError_t launch_fwd(const FwdArgs &a, hipStream_t stream) {
   const int64_t heads = (int64_t)a.batch * a.q_heads;
   const int64_t n128 = ((a.seq_q - 1) / kF4PassRows + 1) * heads,
                 n256 = ((a.seq_q - 1) / 256 + 1) * heads;
-  const bool by_length = a.causal && heads % 8 == 0 &&
-                         (int64_t)a.batch * a.kv_heads * a.seq_k * (2 * kKRowBytes) <= (256 << 20);
+  const int64_t kv_bytes = (int64_t)a.batch * a.kv_heads * a.seq_k * (2 * kKRowBytes);
+  bool by_length = a.causal && heads % 8 == 0 && kv_bytes <= (256 << 20);
   const bool narrow = a.waves == kPPWaves && (n128 <= (by_length ? 2 * a.cus : a.cus) ||
                                               (n256 > a.cus && 113 * n128 < 200 * n256));
+  // 256-row blocks of short sequences do little work on each K and V row: half of
+  // that cache (B48 H16 S448, 176 MB, 126 head by head, 134 by length; B64 Hq32 Hkv8
+  // S768, 201 MB, 562, 600; below, B64 Hq32 Hkv8 S512, 134 MB, level).
+  if (!narrow && a.seq_k < 1024 && kv_bytes > (128 << 20))
+    by_length = false;
   const int rows = a.waves == kR3Waves ? kR3Rows
                    : narrow            ? kF4PassRows
                                        : 32 * kPPWaves;  // 4 waves: two passes of 128

@@ -159,7 +159,7 @@ def test_rejections(wave, dev):
 # Causal blocks by length (24 q heads, a multiple of the 8 XCDs) against head by
 # head (each batch alone: 12): every block is computed alike, so the same bits.
 @pytest.mark.parametrize("out_dt", [1, 2])
-@pytest.mark.parametrize("S", [1, 256, 1000, 3100])
+@pytest.mark.parametrize("S", [1, 256, 385, 1000, 3100])
 def test_blocks_by_length(wave, dev, out_dt, S):
     g = torch.Generator(device=dev).manual_seed(S)
     q, k, v = (torch.randn(2, h, S, 128, generator=g, device=dev) for h in (12, 4, 4))
