@@ -839,9 +839,14 @@ bool half_blocks(int64_t heads, int group, int nb, bool causal, bool by_length, 
 
 // A CTA takes 1.75 us an item (measured) and 4 to start and end; a CU runs one
 // at a time.  Splitting adds the sum kernel: 4 us and 0.06 a CTA (its 128 KiB
-// partial written and read).  Whole blocks on n > CUs: the CUs share the total,
-// and the last blocks run up to half a block's time alone; causal ones by length
-// end with the shortest, and their time is the total's share or the longest.
+// partial written and read; 0.1 with chunks of one item: Hq64 Hkv16 S128, 128 of
+// them, 35.2 against 28.9 whole; Hq32 Hkv8, 64 of them, 26.5 / 28.6).  Whole blocks on
+// n > CUs: the CUs share the total, and the last blocks run up to half a block's time
+// alone; causal ones by length end with the shortest, and their time is the total's
+// share or the longest.
+// So do those of one head an XCD, or of heads that each fill an XCD's CUs, the
+// longest first: Hq64 Hkv8 S8192 3810 whole, 4167 in chunks, B2 Hq64 Hkv8 S4096 2046 /
+// 2205, but S6144 (the longest counts) 2417 / 2341.
 // Candidates: whole blocks, or the shortest chunks for which the CTAs fill the
 // chip once, twice or three times.  B2 Hq16 Hkv4 S2048 causal (128 blocks of 8 to
 // 128 items): whole 229 us, chunks of 43 items (256 CTAs) 105 to 111 and the sum
@@ -871,8 +876,10 @@ KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, bool by_
   };
   KvPlan plan;
   plan.per_head = nkb;
-  double best = by_length ? 4 + 1.75 * std::max((double)longest, (double)total * heads / cus + 2)
-                          : time(heads * nkb, longest);
+  const bool level =
+      by_length || (causal && heads % 8 == 0 && (heads == 8 || nkb >= std::max(cus / 8, 1)));
+  double best = level ? 4 + 1.75 * std::max((double)longest, (double)total * heads / cus + 2)
+                      : time(heads * nkb, longest);
   for (int rounds = 1; split && rounds <= 3; ++rounds) {
     const int64_t most = (int64_t)rounds * cus / heads;
     if (most <= nkb)
@@ -888,7 +895,7 @@ KvPlan kv_plan(int batch, int kv_heads, int group, int nb, bool causal, bool by_
     const int64_t n = per_head(lo);
     if (lo == longest || n == nkb)
       continue;
-    const double t = time(heads * n, lo) + 4 + 0.06 * (double)(heads * n);
+    const double t = time(heads * n, lo) + 4 + (lo == 1 ? 0.1 : 0.06) * (double)(heads * n);
     if (t < best) {
       best = t;
       plan.chunk = lo;
