@@ -6,7 +6,7 @@ import pytest
 import gemm_plan
 from test_gemm_block_gpu import (BLOCK_SHAPES, GRAPH_SHAPES, SPLIT_SHAPES, TILE_SHAPES,
                                  UNALIGNED_SHAPES)
-from test_streamk_gpu import AUTO_SHAPES, auto_workers, short_m_plan
+from test_streamk_gpu import AUTO_SHAPES, FLOAT_SHAPES, auto_workers, short_m_plan
 
 
 def test_split_tags_are_drawn_from_sixty_bits(wave):
@@ -75,6 +75,7 @@ def test_split_shapes_split_every_block(wave):
     assert all(p.splits > 1 for p in plans)
     assert {(p.bm, p.bn) for p in plans} == {(32, 32), (32, 64), (64, 64), (128, 64), (128, 128)}
     assert {p.splits for p in plans} >= {2, 3, 4, 5, 6, 8}
+    assert [auto(wave.runtime.lib(), *s).splits for s in FLOAT_SHAPES] == [2, 4]
     small, large = (auto(wave.runtime.lib(), *s) for s in GRAPH_SHAPES)
     assert small.splits > 1 and large.splits > 1
     top = auto_workers(*GRAPH_SHAPES[0], 256) * 2 * 256 * 256 * 4  # end of its slots

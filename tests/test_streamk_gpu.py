@@ -136,10 +136,10 @@ def test_config3_streamk_bf16(wave, oracle, dev):
 
 # ---- shape-driven dispatch (wave_gemm_auto_launch) ------------------------------
 def auto_workers(M, N, K, cus):
-    """Stream-K workers wave_gemm_auto_launch picks for (M, N, K) on a device
-    with `cus` compute units (0: the tiled or short-M kernel); the rules of
-    auto_workers in 7_amd/csrc/wave_runtime.cpp, restated so the expected
-    choice follows the CU count the device reports."""
+    """Stream-K workers that wave_gemm_auto_launch's workspace holds and its
+    choice of kernel may use for (M, N, K) on a device with `cus` compute units
+    (0: none); the rules of auto_workers in 7_amd/csrc/wave_runtime.cpp, restated
+    so that they follow the CU count the device reports."""
     t = -(-M // 256) * -(-N // 256)
     if M <= 128 or K < 4096 or t >= cus:
         return 0
@@ -154,14 +154,12 @@ def auto_workers(M, N, K, cus):
 
 
 def short_m_plan(M, N, K, cus):
-    """(column block, K splits) of the split short-M kernel
-    wave_gemm_auto_launch picks for (M, N, K), (0, 0) for none; the rules of
-    skinny_split_plan in 7_amd/csrc/gemm_skinny.hip: 64-column blocks when
-    CUs / blocks >= 2, else 128-column ones (2 splits at least when the
-    unsplit kernel's N / 32 CTAs exceed the CUs); at most 4 splits, at least
+    """(columns, K splits) of the partial slots in wave_gemm_auto_launch's
+    workspace for M <= 128, (0, 0) for none; the rules of short_m_workspace in
+    7_amd/csrc/gemm_dispatch.hip: 64 columns when CUs / blocks >= 2, else 128
+    (2 splits at least when N / 32 exceeds the CUs); at most 4 splits, at least
     8 stages of 64 a split; none when a split keeps less than 2048 of K, or
-    less than 4096 where M <= 96 or the unsplit kernel's N / 32 CTAs do not
-    fill the CUs."""
+    less than 4096 where M <= 96 or N / 32 does not fill the CUs."""
     if M > 128 or N < 1024 or K % 64 or K * 2 * 128 >= 2**32 or N * K * 2 >= 2**32:
         return 0, 0
     unsplit = -(-N // 32)
@@ -277,15 +275,15 @@ def test_config3c_auto_dispatch(wave, oracle, dev):
         assert int(ws[sb:].count_nonzero()) == 0
 
 
-# ---- split short-M kernel (wave_gemm_auto_launch, M <= 128) ---------------------
+# ---- K split for M <= 128 (wave_gemm_auto_launch) -------------------------------
 def test_config3a_auto_dispatch(wave, oracle, dev):
     """BASELINE config 3a (128 x 8192 x 8192 bf16) through
-    wave_gemm_auto_launch, the path bench.py reports for it: 128 column
-    blocks of 64, K split in 2 on 256 CUs, partials reduced by each block's
-    last arriver.
+    wave_gemm_auto_launch, the path bench.py reports for it: on 256 CUs 128
+    blocks of 128 x 64, K split in 2, partials reduced by each block's last
+    arriver.
     * N(0,1)/sqrt(K) inputs: every row within 2e-3 * sqrt(K) of the oracle;
-    * bucket inputs: bit-identical to wave_gemm_launch (the unsplit short-M
-      kernel), on a dirty workspace, twice, with the counters back at zero."""
+    * bucket inputs: bit-identical to wave_gemm_launch (unsplit blocks), on a
+      dirty workspace, twice, with the counters back at zero."""
     M, N, K = 128, 8192, 8192
     cus = device_cus(dev)
     bn, s = short_m_plan(M, N, K, cus)
@@ -321,17 +319,16 @@ def test_config3a_auto_dispatch(wave, oracle, dev):
 @pytest.mark.parametrize("in_dt", [1, 2])
 @pytest.mark.parametrize("out_dt,layout", [(torch.float32, "row"), (torch.float16, "col"),
                                            (torch.bfloat16, "row")])
-# On 256 CUs: M from 1 to 128 (waves with no rows skip their MFMAs), N
-# ragged against the column block, K splits of unequal length (131 stages
-# in 4 splits), 64-column blocks in 4, 3 and 2 splits (N 1500, 5000, 8192)
-# and 128-column blocks in 2 (N 11000, 16384, and 24576: 384 CTAs, two
-# rounds); 128 x 4096 x 4096 takes the unsplit kernel (1024 of K a split).
+# On 256 CUs: M from 1 to 128, N ragged against the column block, 64-column
+# blocks with K in 3 and 2 (N 5000, 8192) and 128-column ones with K in 2 (N 11000,
+# 16384); the others unsplit, 24576 with a workspace all the same
+# (test_gemm_plan.py has more splits).
 @pytest.mark.parametrize("shape", [(1, 1024, 8192), (33, 1500, 8384), (100, 8192, 8192),
                                    (100, 11000, 4096), (128, 16384, 4096), (128, 4096, 8192),
                                    (100, 5000, 12288), (128, 24576, 4096), (128, 4096, 4096)])
 def test_split_short_m_matches_unsplit(wave, oracle, dev, in_dt, out_dt, layout, shape):
-    """Bucket inputs make every fp32 sum exact, so the split short-M kernel
-    equals the unsplit one (wave_gemm_launch) bit for bit, on a dirty
+    """Bucket inputs make every fp32 sum exact, so what the workspace lets
+    run (K split or not) equals wave_gemm_launch bit for bit, on a dirty
     workspace, twice in a row."""
     M, N, K = shape
     need = wave.gemm_auto_workspace_bytes(M, N, K)
@@ -397,10 +394,10 @@ def test_split_short_m_alternating_inputs(wave, oracle, dev, shape):
 
 
 def test_split_short_m_graph_replays(wave, oracle, dev):
-    """A captured split short-M launch replays with one fixed counter epoch:
+    """A captured launch for M <= 128 with K split replays with one fixed tag:
     each replay equals wave_gemm_launch's output, with eager launches for
     another B on the same workspace between the replays (every launch leaves
-    the counters at zero, and a word of another epoch counts as zero).  On
+    the counters at zero, and a word of another tag counts as zero).  On
     256 CUs: 64-column blocks in 3 K splits."""
     M, N, K = 100, 5000, 12288
     bn, s = short_m_plan(M, N, K, device_cus(dev))
@@ -445,7 +442,7 @@ def test_split_short_m_shared_workspace_two_shapes(wave, oracle, dev):
     overlap: on 256 CUs the counters of 100 x 5000 x 12288 (3 splits) sit
     inside the fp32 partial slots of 128 x 8192 x 8192 (2 splits), so its
     launches find their counter words holding partial sums the other shape
-    left there.  A word carrying another launch's epoch counts as zero, so
+    left there.  A word without this launch's tag counts as zero, so
     every output equals wave_gemm_launch's, bit for bit (bucket inputs)."""
     cus = device_cus(dev)
     shapes = [(128, 8192, 8192), (100, 5000, 12288)]
@@ -467,11 +464,16 @@ def test_split_short_m_shared_workspace_two_shapes(wave, oracle, dev):
             assert torch.equal(got, ref), (it, j)
 
 
-def test_split_short_m_float_inputs_same_bits(wave, oracle, dev):
+# K split in 2 (M <= 128) and 4 on 256 CUs (test_gemm_plan.py).
+FLOAT_SHAPES = [(96, 8192, 8192), (512, 512, 16384)]
+
+
+@pytest.mark.parametrize("shape", FLOAT_SHAPES)
+def test_split_short_m_float_inputs_same_bits(wave, oracle, dev, shape):
     """Inexact inputs, fp32 C: the last arriver sums the partials in split
     order whichever arrives last, so every launch gives the same bits, within
     2e-3 * sqrt(K) of the oracle."""
-    M, N, K = 96, 4096, 8192
+    M, N, K = shape
     g = torch.Generator(device="cpu").manual_seed(41)
     a = (torch.randn((M, K), generator=g) / np.sqrt(K)).to(torch.float16)
     b = (torch.randn((N, K), generator=g) / np.sqrt(K)).to(torch.float16)
