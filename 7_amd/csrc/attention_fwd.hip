@@ -25,7 +25,7 @@ hipError_t launch_fwd(const FwdArgs &a, hipStream_t stream) {
   p.seq_k = a.seq_k;
   // The default (8 waves a 256-row block, one CTA a CU) gives way to the 4-wave
   // kernel on 128-row blocks where those are at most one a CU (half as many
-  // 256-row ones would leave CUs idle: B1 Hq32 Hkv8 S1000 causal bf16 32.7 -> 26.0
+  // 256-row ones would leave CUs idle: B1 Hq32 Hkv8 S1000 causal bf16 30.1 -> 25.2
   // us, B1 H8 S512 16.8 -> 13.0, B1 H16 S1024 28.8 -> 23.1; at 384 blocks of 128
   // the 8-wave kernel is ahead, 24.8 / 28.0), or where, on more than one
   // round of 256-row blocks, they save more padded rows than their rate costs
@@ -42,8 +42,8 @@ hipError_t launch_fwd(const FwdArgs &a, hipStream_t stream) {
   // 2228.  In long and short pairs the 4-wave kernel's blocks are ahead up to two
   // of them a CU: B2 Hq16 Hkv4 S2048 59 (8-wave, head by head), 53 (8-wave, by
   // length), 47 (pairs); B1 H16 S4096 103, 98, 91; with four a CU B1 Hq64 Hkv8
-  // S2048 114, 77, 82.  One block a CU has nothing to order (B1 Hq32 Hkv8 S1000
-  // 23.4 head by head, 24.1 by length).
+  // S2048 114, 77, 82.  One block a CU has nothing to order (B1 Hq32 Hkv8 S1000 3 %
+  // slower by length).
   const int64_t heads = (int64_t)a.batch * a.q_heads;
   const int64_t n128 = ((a.seq_q - 1) / kF4PassRows + 1) * heads,
                 n256 = ((a.seq_q - 1) / 256 + 1) * heads;

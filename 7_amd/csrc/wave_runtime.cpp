@@ -207,9 +207,9 @@ int device_cus(int *cus) {
   return WAVE_OK;
 }
 
-// Stream-K workers the shape-driven dispatch uses for (M, N, K), or 0 for
-// the tiled path: fewer 256x256 tiles than CUs, K >= 4096 (64 K units a
-// tile), M > 128 (the short-M kernel's range).
+// Stream-K workers the shape-driven dispatch offers gemm_plan for (M, N, K), or
+// 0 for none: fewer 256x256 tiles than CUs, K >= 4096 (64 K units a tile),
+// M > 128 (below, blocks and short_m_workspace).
 int auto_workers(int M, int N, int K, int cus) {
   const int64_t tiles = (int64_t)wave::gemm::tiles_for(M) * wave::gemm::tiles_for(N);
   if (M <= 128 || K < 4096 || tiles >= cus)

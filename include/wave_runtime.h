@@ -305,7 +305,7 @@ int wave_fa_bwd_launch(const void *Q, const void *K, const void *V, const void *
  * launch in flight), which lets the dK/dV kernel cut its key blocks' work into
  * chunks for several CTAs where the blocks are fewer than the CUs or causal
  * ones of uneven length; wave_fa_bwd_workspace_bytes gives its size (0 where
- * whole blocks are used).  A smaller one (or none) runs whole blocks. */
+ * whole blocks are used, at most 128 KiB for three CTAs a CU: 96 MiB on 256).  A smaller one (or none) runs whole blocks. */
 int wave_fa_bwd_workspace_bytes(int batch, int q_heads, int kv_heads, int seq, int causal,
                                 size_t *bytes);
 int wave_fa_bwd_workspace_launch(const void *Q, const void *K, const void *V, const void *O,
