@@ -808,13 +808,13 @@ struct KvPlan {
 // number nb of them.  128-key blocks spend half of the last one on keys past the
 // sequence, one CTA a CU; 64-key ones run two a CU, with more LDS traffic an item.
 // us a CTA to start and end, and an item, fitted to 130 measured shapes: 3.6 (3.3
-// in many rounds) and 1.75; 1.1 and 2.07 (alone on its CU), 2.85 and 2.5 (two a CU).  Causal blocks by
-// length end level (0.86, but the longest come in whole rounds); head by head, two
-// or four lengths in turn fall on the same CUs each time (1.25 over many rounds).
-// The backward (us, 128-key / 64-key): S64 B32 H16 32.9 / 26.3, B256 H16 247 / 208,
-// B1 H8 15.5 / 13.8, Hq64 Hkv1 130 / 154; S192 B24 H12 62.5 / 54.5, B128 Hq16 Hkv2
-// 254 / 282; S320 B32 H16 180 / 188; causal S448 B64 H16 534 / 488, S960 B32 H16 745
-// / 758.
+// in many rounds) and 1.75; 1.1 and 2.07 (alone on its CU), 2.85 and 2.5 (two a CU).
+// Causal blocks by length end level (0.86, but the longest come in whole rounds);
+// head by head, two or four lengths in turn fall on the same CUs each time (1.25 over
+// many rounds).  The backward (us, 128-key / 64-key): S64 B32 H16 32.9 / 26.3, B256
+// H16 247 / 208, B1 H8 15.5 / 13.8, Hq64 Hkv1 130 / 154; S192 B24 H12 62.5 / 54.5,
+// B128 Hq16 Hkv2 254 / 282; S320 B32 H16 180 / 188; causal S448 B64 H16 534 / 488,
+// S960 B32 H16 745 / 758.
 bool half_blocks(int64_t heads, int group, int nb, bool causal, bool by_length, int cus) {
   const int nkb = (nb + 1) / 2;
   const double longest = (double)group * nb, mean = (double)group * nkb;  // causal: of a block

@@ -292,7 +292,7 @@ def _eager_device_tensor(x: torch.Tensor) -> bool:
     that its pointer is what the operation runs on and what lies there are its
     values (a lazily negated view's are not; a zero tensor has no memory)."""
     return (x.is_cuda and type(x) in (torch.Tensor, torch.nn.Parameter)
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch.compiler.is_compiling() and not torch._C._is_tracing()
             and not torch._C._functorch.is_functorch_wrapped_tensor(x)
             and torch._C._len_torch_dispatch_stack() == 0
             and not x.is_neg() and not x._is_zerotensor())
