@@ -13,11 +13,15 @@
 // round the probabilities otherwise: results 2e-4 away.)
 //
 // Nothing here is near a rate of the chip: a round is a chain of load -> QK ->
-// maxima -> exp2 -> PV steps, and the next round's loads are in flight during it.
-// Measured (us, one workgroup / this grid): 64 queries x 1024 keys x 64 130 / 8.5
-// (8 CTAs x 16 waves), 16 x 4096 x 128 957 / 36.5, 4096 x 2048 x 128 11700 / 30.
-// Keeping the query fragments in LDS lets the D = 128 step fit 128 registers
-// (with them in registers it spilled: 16 x 4096 x 128 47.8; 64 x 1024 x 64 10.9).
+// maxima -> exp2 -> PV steps, with the next round's loads in flight, and four waves
+// share a SIMD's VALU.  Measured (us, one workgroup / this grid): 64 queries x 1024
+// keys x 64 130 / 7.9 (8 CTAs x 16 waves), 16 x 4096 x 128 957 / 35.5, 4096 x 2048 x
+// 128 11700 / 29.  Keeping the query fragments in LDS lets the D = 128 step fit 128
+// registers (in registers it spilled: 16 x 4096 x 128 47.8, 64 x 1024 x 64 10.9);
+// maxima without LDS shuffles and masks, and the exp2 instruction for P, took 64 x
+// 1024 x 64 from 8.4 to 7.9 and 1 x 4096 x 16 from 19.1 to 16.1; rounds of even length
+// 64 x 600 x 48 from 5.8 to 5.3; V gathered a round ahead 64 x 1024 x 63 from 29.2 to
+// 26.5.
 #include "attention.hpp"
 #include "fa_small.hpp"
 
@@ -33,6 +37,18 @@ constexpr int kSplitWaves = 16;
 // ND: 32-wide steps of the head dimension held in registers (D <= 32 ND, D a
 // multiple of 8, 16-byte aligned rows), or 0 for any D and alignment.
 // TC: 16-column tiles a CTA owns.
+// Largest of the four lanes l % 16 + 16 {0..3}, in all of them: rows of 16 lanes
+// exchanged by the VALU (an xor shuffle goes through LDS and takes seven more
+// instructions).
+__device__ __forceinline__ float rows_max4(float v) {
+  const uint32_t a = __builtin_bit_cast(uint32_t, v);
+  const auto x = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+  v = fmaxf(__builtin_bit_cast(float, (uint32_t)x[0]), __builtin_bit_cast(float, (uint32_t)x[1]));
+  const uint32_t b = __builtin_bit_cast(uint32_t, v);
+  const auto y = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)y[0]), __builtin_bit_cast(float, (uint32_t)y[1]));
+}
+
 template <int TC> constexpr int max_waves() { return TC > 2 ? kSplitWaves / 2 : kSplitWaves; }
 
 template <int ND, int TC>
@@ -89,32 +105,34 @@ __global__ __launch_bounds__(64 * max_waves<TC>()) void small_split_kernel(
       }
     }
   };
-  auto load_v = [&](int n0) {
-    if constexpr (ND > 0) {
-#pragma unroll
-      for (int i = 0; i < TC; ++i) {
-        const int piece = lane + 64 * i, key = n0 + piece / (2 * TC);
-        vf[i] = chunk(rv, seq_n, key, c0 + 8 * (piece % (2 * TC)));
-      }
-    }
-  };
   auto key_of = [&](int n0, int j) { return n0 + (j < 4 ? 4 * grp + j : 16 + 4 * grp + j - 4); };
-  auto store_v = [&](int n0) {
+  uint32_t vr[ND > 0 ? 1 : TC][8];  // ND = 0: the operands' halves, gathered
+  auto load_v = [&](int n0) {
 #pragma unroll
     for (int i = 0; i < TC; ++i) {
       if constexpr (ND > 0) {
-        sv[wave][i][lane] = __builtin_bit_cast(f32x4, vf[i]);
+        const int piece = lane + 64 * i, key = n0 + piece / (2 * TC);
+        vf[i] = chunk(rv, seq_n, key, c0 + 8 * (piece % (2 * TC)));
       } else {
         const int c = c0 + 16 * i + col;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          vr[i][j] = vh[(size_t)min(key_of(n0, j), seq_n - 1) * D + min(c, D - 1)];
+      }
+    }
+  };
+  auto store_v = [&](int n0) {
+#pragma unroll
+    for (int i = 0; i < TC; ++i) {
+      if constexpr (ND == 0) {
+        const bool in = c0 + 16 * i + col < D;
         u32x4 w = zero4;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int key = key_of(n0, j);
-          const uint32_t x = vh[(size_t)min(key, seq_n - 1) * D + min(c, D - 1)];
-          w[j >> 1] |= (key < seq_n && c < D ? x : 0u) << (16 * (j & 1));
-        }
-        sv[wave][i][lane] = __builtin_bit_cast(f32x4, w);
+        for (int j = 0; j < 8; ++j)
+          w[j >> 1] |= (in && key_of(n0, j) < seq_n ? vr[i][j] : 0u) << (16 * (j & 1));
+        vf[i] = w;
       }
+      sv[wave][i][lane] = __builtin_bit_cast(f32x4, vf[i]);
     }
   };
   // V^T of block b of the round as the PV product's A operand: column c0 + 16t +
@@ -152,7 +170,8 @@ __global__ __launch_bounds__(64 * max_waves<TC>()) void small_split_kernel(
     }
   }
   load_k(32 * wave);
-  load_v(32 * wave);
+  if (ND > 0 || wave < blocks)
+    load_v(32 * wave);
   if constexpr (ND > 0) {
     if (wave == 0) {
 #pragma unroll
@@ -194,31 +213,48 @@ __global__ __launch_bounds__(64 * max_waves<TC>()) void small_split_kernel(
       }
       load_k(n0 + 32 * W);  // the next round's, early; zeros past the last key
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        p[j] = key_of(n0, j) < seq_n ? s[j >> 2][j & 3] : -__builtin_inff();
-        top = fmaxf(top, p[j]);
+      for (int j = 0; j < 8; ++j)
+        p[j] = s[j >> 2][j & 3];
+      if (n0 + 31 >= seq_n) {  // the last block
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          p[j] = key_of(n0, j) < seq_n ? p[j] : -__builtin_inff();
       }
-      top = small_wave_max4(top);
-      if (grp == 0)
-        smax[col][wave] = top;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        top = fmaxf(top, p[j]);
+      top = rows_max4(top);
     }
+    if (grp == 0)
+      smax[col][wave] = top;  // -inf without a block
     lds_barrier();  // the round's maxima; the last round's chain is done
     float before = m;
 #pragma unroll
     for (int w4 = 0; w4 < MAXW; w4 += 4) {
+      if (w4 >= W)
+        break;
       const f32x4 x = *reinterpret_cast<const f32x4 *>(&smax[col][w4]);
+      if (w4 + 4 <= wave) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        before = fmaxf(before, w4 + i < wave ? x[i] : -__builtin_inff());
-        m = fmaxf(m, w4 + i < here ? x[i] : -__builtin_inff());
+        for (int i = 0; i < 4; ++i)
+          before = fmaxf(before, x[i]);
+      } else if (w4 < wave) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          before = fmaxf(before, w4 + i < wave ? x[i] : -__builtin_inff());
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        m = fmaxf(m, w4 + i < W ? x[i] : -__builtin_inff());
     }
     if (mine) {
       const float m_new = fmaxf(before, top);
       float psum = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        p[j] = exp2f(p[j] - m_new);
+        // Below 2^-126 the instruction gives 0 where exp2f is subnormal: nothing in
+        // f16, nor in a row's sum, one of whose terms is 1.
+        p[j] = __builtin_amdgcn_exp2f(p[j] - m_new);
         psum += p[j];
       }
       sp[wave][lane] = u32x4{small_pack_f16(p[0], p[1]), small_pack_f16(p[2], p[3]),
@@ -227,7 +263,8 @@ __global__ __launch_bounds__(64 * max_waves<TC>()) void small_split_kernel(
       if (grp == 0)
         salpha[wave][col] = exp2f(before - m_new);
       store_v(n0);
-      load_v(n0 + 32 * W);
+      if (ND > 0 || wave < blocks - b0 - W)
+        load_v(n0 + 32 * W);
     }
     lds_barrier();  // the round's P, V, sums and factors
     if (carries) {
@@ -252,7 +289,7 @@ __global__ __launch_bounds__(64 * max_waves<TC>()) void small_split_kernel(
                                                        0);
         }
       };
-      constexpr int G = ND == 4 && TC == 2 ? 2 : 4;  // what the registers hold
+      constexpr int G = 4;
       int b = 0;
 #pragma unroll 1
       for (; b + G <= here; b += G)
@@ -279,7 +316,9 @@ template <int TC>
 hipError_t launch_tc(const _Float16 *Q, const _Float16 *K, const _Float16 *V, float *O, int block_m,
                      int seq_n, int D, hipStream_t stream) {
   const int blocks = (seq_n - 1) / 32 + 1, most = max_waves<TC>();
-  const int waves = blocks < TC ? TC : blocks < most ? blocks : most;
+  // Rounds of even length.
+  const int rounds = (blocks - 1) / most + 1, even = (blocks - 1) / rounds + 1;
+  const int waves = even < TC ? TC : even;
   const int col_units = (D - 1) / (16 * TC) + 1;
   // At most 2^27 units (block_m * D < 2^31); a grid dimension holds fewer than 2^32
   // threads.
@@ -289,15 +328,20 @@ hipError_t launch_tc(const _Float16 *Q, const _Float16 *K, const _Float16 *V, fl
   const uintptr_t at = reinterpret_cast<uintptr_t>(Q) | reinterpret_cast<uintptr_t>(K) |
                        reinterpret_cast<uintptr_t>(V);
   const bool vec = D % 8 == 0 && at % 16 == 0 && rows * D < (1 << 30);
-  if (vec && D <= 64)
-    hipLaunchKernelGGL((small_split_kernel<2, TC>), grid, block, 0, stream, Q, K, V, O, block_m,
-                       seq_n, D, col_units, units);
-  else if (vec && D <= 128)
-    hipLaunchKernelGGL((small_split_kernel<4, TC>), grid, block, 0, stream, Q, K, V, O, block_m,
-                       seq_n, D, col_units, units);
+  auto go = [&](auto nd) {
+    hipLaunchKernelGGL((small_split_kernel<decltype(nd)::value, TC>), grid, block, 0, stream, Q, K,
+                       V, O, block_m, seq_n, D, col_units, units);
+  };
+  if (!vec || D > 128)
+    go(std::integral_constant<int, 0>{});
+  else if (D <= 32)
+    go(std::integral_constant<int, 1>{});
+  else if (D <= 64)
+    go(std::integral_constant<int, 2>{});
+  else if (D <= 96)
+    go(std::integral_constant<int, 3>{});
   else
-    hipLaunchKernelGGL((small_split_kernel<0, TC>), grid, block, 0, stream, Q, K, V, O, block_m,
-                       seq_n, D, col_units, units);
+    go(std::integral_constant<int, 4>{});
   return hipGetLastError();
 }
 

@@ -93,6 +93,19 @@ def test_rounds_as_one_running_max(wave, dev, M, S, D, ramp):
     assert ((o - ref).norm() / ref.norm()).item() < 6e-5
 
 
+@pytest.mark.parametrize("D", [32, 64, 96, 100])
+def test_scores_far_apart(wave, dev, D):
+    """Blocks whose scores lie hundreds apart, rising and falling: factors and
+    probabilities down to zero (below 2^-126 and to 2^-149 among them)."""
+    q, k, v = inputs(48, 900, D, dev, 8)
+    k *= ((torch.arange(900, device=dev) // 40 * 5 % 7).half() * 12)[:, None]
+    o = wave.flash_attention_f32(q, k, v).double()
+    ref = in_key_order(q, k, v)
+    assert bool(o.isfinite().all())
+    # A score of up to 2^9 carries an fp32 error of 2^-13, and so does its power.
+    assert ((o - ref).norm() / ref.norm()).item() < 2e-4
+
+
 def test_excluded_leading_block_is_nan(wave, dev):
     """With every score of the first 32 keys at -inf the running max starts at
     -inf and the row is NaN, as in one pass over the keys."""
